@@ -120,6 +120,19 @@ __device__ __forceinline__ T expmi_phase(float t) {
 }
 #endif
 
+// Loads of phase factors and angles.  Arrays as large as the eight L2s
+// together (32 MB) are read once a pass and never met again in a cache: they
+// are loaded nontemporally, which leaves the state there (24 qubits: a pass
+// with three phases 179 -> 165 us).  Smaller ones stay cached for the other
+// states of a batch.
+template <typename V> __device__ __forceinline__ V ldp(const GL V* p) {
+#if UA_STREAM_PHASES
+  return __builtin_nontemporal_load(p);
+#else
+  return *p;
+#endif
+}
+
 // Two consecutive elements (aligned to two elements), as native vectors.
 #if UA_DOUBLE
 typedef double v2r __attribute__((ext_vector_type(2)));
@@ -132,7 +145,12 @@ __device__ __forceinline__ void st2(GL T* p, T a, T b) {
   *reinterpret_cast<GL v2r*>(p) = x; *reinterpret_cast<GL v2r*>(p + 1) = y;
 }
 __device__ __forceinline__ void ld2r(const GL R* p, R& a, R& b) {
-  const v2r x = *reinterpret_cast<const GL v2r*>(p); a = x.x; b = x.y;
+  const v2r x = ldp(reinterpret_cast<const GL v2r*>(p)); a = x.x; b = x.y;
+}
+__device__ __forceinline__ void ld2f(const GL T* p, T& a, T& b) {
+  const v2r x = ldp(reinterpret_cast<const GL v2r*>(p));
+  const v2r y = ldp(reinterpret_cast<const GL v2r*>(p + 1));
+  a = cmk(x.x, x.y); b = cmk(y.x, y.y);
 }
 #else
 typedef float v4r __attribute__((ext_vector_type(4)));
@@ -146,11 +164,16 @@ __device__ __forceinline__ void st2(GL T* p, T a, T b) {
   *reinterpret_cast<GL v4r*>(p) = x;
 }
 __device__ __forceinline__ void ld2r(const GL R* p, R& a, R& b) {
-  const v2r x = *reinterpret_cast<const GL v2r*>(p); a = x.x; b = x.y;
+  const v2r x = ldp(reinterpret_cast<const GL v2r*>(p)); a = x.x; b = x.y;
+}
+__device__ __forceinline__ void ld2f(const GL T* p, T& a, T& b) {
+  const v4r x = ldp(reinterpret_cast<const GL v4r*>(p));
+  a = cmk(x.x, x.y); b = cmk(x.z, x.w);
 }
 #endif
 
 // ---- gates on a thread's cube of 16 amplitudes (cube bits 0..3)
+#if !UA_MFMA
 template <int B>
 __device__ __forceinline__ void cube_1q(T (&c)[16], const SC R* u) {
   const T u00 = ldc(u, 0), u01 = ldc(u, 1), u10 = ldc(u, 2), u11 = ldc(u, 3);
@@ -184,6 +207,82 @@ __device__ __forceinline__ void cube_2q(T (&c)[16], const SC R* u) {
     for (int s = 0; s < 4; ++s) c[idx[s]] = o[s];
   }
 }
+#else
+// Gates on the matrix cores as lane-private products:
+// v_mfma_f32_4x4x1 with 16 blocks gives lane l
+//   acc[r] += A(r) * B(l), r = 0..3, with A(r) taken from lane 4 (l / 4) + r,
+// so with A the same in every block each lane multiplies its own column by
+// one column of a 4-row matrix, 4 FMAs per lane at twice the vector units'
+// rate (123-144 against 70-76 TFLOP/s measured), with each product rounded
+// as fmaf rounds it.  A 1-qubit gate is the 4x4 real block
+//   [Re -Im; Im Re] over (Re x, Im x, Re y, Im y):
+// four of them for each amplitude pair.  The instruction ignores the lane
+// mask: every lane of a wavefront takes part (whole workgroups, no branch).
+__device__ __forceinline__ v4r mfma4(float a, float b, v4r c) {
+  return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+// this lane's real row (Re or Im, by its lowest bit) of complex entry u
+__device__ __forceinline__ void row_of(T u, bool im, float& re_col, float& im_col) {
+  re_col = im ? u.y : u.x;
+  im_col = im ? u.x : -u.y;
+}
+template <int B>
+__device__ __forceinline__ void cube_1q(T (&c)[16], const SC R* u) {
+  const bool im = threadIdx.x & 1, low = threadIdx.x & 2;
+  float a[4];
+  row_of(csel(low, ldc(u, 2), ldc(u, 0)), im, a[0], a[1]);
+  row_of(csel(low, ldc(u, 3), ldc(u, 1)), im, a[2], a[3]);
+  v4r acc[8];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int j = ((q >> B) << (B + 1)) | (q & ((1 << B) - 1));
+      const T x = c[(s & 2) ? j | (1 << B) : j];
+      acc[q] = mfma4(a[s], (s & 1) ? x.y : x.x, s == 0 ? v4r{0.f, 0.f, 0.f, 0.f} : acc[q]);
+    }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int j = ((q >> B) << (B + 1)) | (q & ((1 << B) - 1));
+    c[j] = cmk(acc[q].x, acc[q].y);
+    c[j | (1 << B)] = cmk(acc[q].z, acc[q].w);
+  }
+}
+// gate index bit 1 = cube bit B1, bit 0 = cube bit B0: the 8x8 real block, rows
+// of gate entries 0, 1 and of 2, 3 as two 4-row products
+template <int B1, int B0>
+__device__ __forceinline__ void cube_2q(T (&c)[16], const SC R* u) {
+  constexpr int lo = B0 < B1 ? B0 : B1, hi = B0 < B1 ? B1 : B0;
+  const bool im = threadIdx.x & 1, low = threadIdx.x & 2;
+  v4r acc[2][4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float ar, ai;
+      row_of(csel(low, ldc(u, (2 * t + 1) * 4 + s), ldc(u, 2 * t * 4 + s)), im, ar, ai);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          int j = ((q >> lo) << (lo + 1)) | (q & ((1 << lo) - 1));
+          j = ((j >> hi) << (hi + 1)) | (j & ((1 << hi) - 1));
+          const T x = c[j | ((s & 1) << B0) | ((s >> 1) << B1)];
+          acc[t][q] = mfma4(h ? ai : ar, h ? x.y : x.x,
+                            s + h == 0 ? v4r{0.f, 0.f, 0.f, 0.f} : acc[t][q]);
+        }
+    }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    int j = ((q >> lo) << (lo + 1)) | (q & ((1 << lo) - 1));
+    j = ((j >> hi) << (hi + 1)) | (j & ((1 << hi) - 1));
+    c[j] = cmk(acc[0][q].x, acc[0][q].y);
+    c[j | (1 << B0)] = cmk(acc[0][q].z, acc[0][q].w);
+    c[j | (1 << B1)] = cmk(acc[1][q].x, acc[1][q].y);
+    c[j | (1 << B1) | (1 << B0)] = cmk(acc[1][q].z, acc[1][q].w);
+  }
+}
+#endif
 // CZ with both qubits on cube bits A, B
 template <int A, int B>
 __device__ __forceinline__ void negate_cc(T (&c)[16]) {
@@ -309,7 +408,15 @@ std::string generate(const PassShape& ps) {
   const bool dbl = ps.dtype == UA_COMPLEX128;
   const int tbits = p.tile_bits;              // 12..14: 2^(tbits-4) threads of 16 amplitudes
   const int threads = 1 << (tbits - 4);
-  s << "#define UA_DOUBLE " << (dbl ? 1 : 0) << "\n" << kPrelude;
+  // complex64 passes of 13- and 14-bit tiles: gates on the matrix cores.  With
+  // phase factors read past the caches as well, the 9 passes of a 24-qubit,
+  // 200-gate circuit went from 1155 to 1060 us (without the latter 1147);
+  // what is left is memory traffic (the same passes without
+  // gates: 950).  12-bit passes keep the vector FMAs: there the gain was 2 %
+  // of a gradient step, and they round as the interpreted passes do.
+  const bool mfma = !dbl && tbits > 12;
+  s << "#define UA_DOUBLE " << (dbl ? 1 : 0) << "\n#define UA_MFMA " << (mfma ? 1 : 0)
+    << "\n#define UA_STREAM_PHASES " << (n >= (dbl ? 21 : 22) ? 1 : 0) << "\n" << kPrelude;
   const int waves = dbl ? 2 : (g_compiled_waves > 0 ? int(g_compiled_waves) : 4);
   s << "extern \"C\" __global__ __launch_bounds__(" << threads
     << ") __attribute__((amdgpu_waves_per_eu("
@@ -360,7 +467,7 @@ std::string generate(const PassShape& ps) {
             e << "      " << x0 << " = cmul(pf" << o << "[" << 2 * pk << "], " << x0 << "); "
               << x1 << " = cmul(pf" << o << "[" << 2 * pk + 1 << "], " << x1 << ");\n";
           else
-            e << "      { T f0, f1; ld2((const GL T*)ops[" << o << "].data + b * ops[" << o
+            e << "      { T f0, f1; ld2f((const GL T*)ops[" << o << "].data + b * ops[" << o
               << "].bstride + g, f0, f1); " << x0 << " = cmul(f0, " << x0 << "); " << x1
               << " = cmul(f1, " << x1 << "); }\n";
           break;
@@ -414,7 +521,7 @@ std::string generate(const PassShape& ps) {
       if (ps.ops[o].kind != UA_FOP_PHASE_FACTORS) continue;
       s << "  T pf" << o << "[16];\n";
       for (int k = 0; k < 8; ++k)
-        s << "  ld2((const GL T*)ops[" << o << "].data + b * ops[" << o << "].bstride + (origin | "
+        s << "  ld2f((const GL T*)ops[" << o << "].data + b * ops[" << o << "].bstride + (origin | "
           << hex64(depk[k]) << " | dep_t), pf" << o << "[" << 2 * k << "], pf" << o << "["
           << 2 * k + 1 << "]);\n";
     }

@@ -201,3 +201,24 @@ def test_compiled_tile_sizes(device, n, tile_bits):
     out = prog.run(torch.from_numpy(psi).to(device, torch.complex64)).cpu().numpy()
     assert rel_err(out, ref) < 1e-4
     assert np.max(U.fidelity_error(ref, out)) < 1e-5
+
+
+@pytest.mark.parametrize("n,batch", [(13, 2), (14, 1)])
+def test_compiled_every_gate_of_a_cube(device, n, batch):
+    """1-qubit gates on each cube bit and 2-qubit gates on every ordered pair
+    of them, in one stage of a 13-bit tile (complex64: lane-private matrix-core
+    products).  16 gates of at most 8 rounded terms each: 16 * 8 * 2^-24 =
+    7.7e-6 of the largest amplitude's group."""
+    from unitair_amd.circuits import Circuit, Gate
+    rng = np.random.default_rng(41)
+    low = [n - 1 - b for b in range(4)]              # the qubits of index bits 0..3
+    gates = [Gate("dense", (q,), matrix=haar_unitary(2, rng)) for q in low]
+    gates += [Gate("dense", (a, b), matrix=haar_unitary(4, rng))
+              for a in low for b in low if a != b]
+    prog = FusedProgram(Circuit(n, gates), device=device, reorder=False, merge_1q=False,
+                        compiled=True)
+    assert prog.num_passes == 1 and prog.num_compiled == 1
+    psi = seeded_state_np(n, (batch,), seed=5)
+    ref = np.stack([oc.run_closed_form(gates, p) for p in psi])
+    out = prog.run(torch.from_numpy(psi).to(device, torch.complex64)).cpu().numpy()
+    assert rel_err(out, ref) < 1e-5
