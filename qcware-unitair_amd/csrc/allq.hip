@@ -6,11 +6,12 @@
 // The reference loops over qubits with swap (a transposed view) + einsum and
 // finishes with a permute/roll and a contiguous copy: one pass over the state
 // per qubit plus the copy.  Gates on distinct qubits commute, so here they are
-// grouped into tiled passes.  A workgroup loads a tile of 2^TB amplitudes into
-// LDS (TB = 12, or 13 for complex64 where that saves a pass); the tile spans
-// TB index bits ("local bits").  In up to four stages every thread holds a
-// cube of 16 amplitudes over 4 of the local bits and applies each target
-// bit's 2x2 matrix in registers.
+// grouped into tiled passes.  A workgroup owns a tile of 2^TB amplitudes (TB =
+// 12, or 13 for complex64 where that saves a pass); the tile spans TB index
+// bits ("local bits").  In up to four stages every thread holds a cube of 16
+// amplitudes over 4 of the local bits and applies each target bit's 2x2 matrix
+// in registers; the tile passes from stage to stage through LDS, while the
+// first and the last stage read and write the state directly.
 //
 // Every tile keeps the lowest R state bits (R = 2 for complex64, 1 for
 // complex128: runs of at least 32 bytes) and takes up to TB - R target bits;
@@ -25,10 +26,16 @@
 // with the dense kernels.
 //
 // Cost: each gate is 8 FMAs per amplitude, so a layer of g gates on 2^n
-// amplitudes is g * 8 * 2^n FMAs on the vector units; apply_all_qubits at 24
-// qubits (3.2e9 FMAs) is bound by them (82 us at the FP32 vector peak)
-// rather than by its two passes over HBM.
-#include "ua_common.h"
+// amplitudes is g * 8 * 2^n FMAs.  On the vector units that bound complex64
+// layers (apply_all_qubits at 24 qubits: 3.2e9 FMAs, 82 us at their peak); as
+// lane-private matrix-core products they take half of it and run beside the
+// address arithmetic, and with the two trips through LDS saved the call went
+// from 184 to 161 us.  Now the two passes' memory phases bound it: without
+// any gate they take 57 us (contiguous tiles, out of place) and 75 us (32-byte
+// runs, in place).  Measured slower and not kept: persistent workgroups that
+// load their next tile ahead (189 us; 160 against 136 us without gates), and
+// 64-byte runs (three passes, 174 us).
+#include "mfma_common.h"
 
 namespace ua {
 int apply_operator_impl(void* out, const void* state, const void* op, int dtype, int n,
@@ -63,16 +70,43 @@ __device__ __forceinline__ T cmul(T a, T b) {
   return r;
 }
 
-template <int B, typename T>
-__device__ __forceinline__ void cube_1q(T (&c)[kCube], const T u00, const T u01, const T u10,
-                                        const T u11) {
+template <int B>
+__device__ __forceinline__ void cube_1q(double2 (&c)[kCube], const double2 u00,
+                                        const double2 u01, const double2 u10,
+                                        const double2 u11) {
 #pragma unroll
   for (int j = 0; j < kCube; ++j) {
     if (j & (1 << B)) continue;
     const int k = j | (1 << B);
-    const T a = c[j], b = c[k];
+    const double2 a = c[j], b = c[k];
     c[j] = cmad(cmul(u00, a), u01, b);
     c[k] = cmad(cmul(u10, a), u11, b);
+  }
+}
+// complex64: lane-private matrix-core products (mfma_common.h).  The gate is
+// the 4x4 real block [Re -Im; Im Re] over (Re a, Im a, Re b, Im b); lane l
+// holds row l % 4 of it, and each amplitude pair takes four products.
+template <int B>
+__device__ __forceinline__ void cube_1q(float2 (&c)[kCube], const float2 u00, const float2 u01,
+                                        const float2 u10, const float2 u11) {
+  const bool im = threadIdx.x & 1, low = threadIdx.x & 2;
+  const float2 ua = low ? u10 : u00, ub = low ? u11 : u01;
+  const float row[4] = {im ? ua.y : ua.x, im ? ua.x : -ua.y, im ? ub.y : ub.x,
+                        im ? ub.x : -ub.y};
+  floatx4 acc[8];
+#pragma unroll
+  for (int s = 0; s < 4; ++s)
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int j = ((q >> B) << (B + 1)) | (q & ((1 << B) - 1));
+      const float2 x = c[(s & 2) ? j | (1 << B) : j];
+      acc[q] = mfma4(row[s], (s & 1) ? x.y : x.x, s == 0 ? floatx4{0.f, 0.f, 0.f, 0.f} : acc[q]);
+    }
+#pragma unroll
+  for (int q = 0; q < 8; ++q) {
+    const int j = ((q >> B) << (B + 1)) | (q & ((1 << B) - 1));
+    c[j] = make_float2(acc[q][0], acc[q][1]);
+    c[j | (1 << B)] = make_float2(acc[q][2], acc[q][3]);
   }
 }
 
@@ -114,65 +148,54 @@ struct AllqPass {
 };
 
 template <typename T, int TB>
-__global__ __launch_bounds__((1 << TB) / kCube) void allq_pass_kernel(T* out, const T* in,
-                                                                      const T* __restrict__ op,
-                                                                      AllqPass a) {
+__global__ __launch_bounds__((1 << TB) / kCube) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 2)))
+void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a) {
   constexpr int kTile = 1 << TB;
-  constexpr int kThreads = kTile / kCube;
-  constexpr int kTidBits = TB - 4;
   __shared__ T tile[kTile];
   const int tid = threadIdx.x;
   const int64_t N = int64_t(1) << a.n;
-
-  // Element pair e = 2*tid + 2*kThreads*k of a tile (k = 0..7).  Tile bit 0
-  // is state bit 0, so the pair is contiguous in memory; tile bits 1..TB-4
-  // come from the thread index and the top three from k.
-  uint64_t dep_t = 0;
-#pragma unroll
-  for (int i = 1; i <= kTidBits; ++i) dep_t |= uint64_t(((2 * tid) >> i) & 1) << a.local[i];
-  uint64_t dep_k[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    dep_k[k] = 0;
-#pragma unroll
-    for (int i = TB - 3; i < TB; ++i)
-      dep_k[k] |= uint64_t((k >> (i - (TB - 3))) & 1) << a.local[i];
-  }
   // One tile per workgroup.  XCD order: workgroups are dealt to the 8 XCDs
   // round-robin, so workgroup w takes tile (w % 8) * (tiles / 8) + w / 8 and
   // each XCD walks a contiguous range of tiles.
   int64_t tg = blockIdx.x;
   if (tg >= a.total_tiles) return;
   if (a.xcd_order) tg = (tg & 7) * (a.total_tiles >> 3) + (tg >> 3);
-  auto origin_of = [&](int64_t t, int64_t bstride) -> int64_t {
-    const int64_t b = t >> a.log2_tiles;
-    const uint64_t tis = uint64_t(t) & ((uint64_t(1) << a.log2_tiles) - 1);
-    return b * bstride + int64_t(insert_zero_bits(tis, a.local, TB) | dep_t);
-  };
-  {
-    const T* src = in + origin_of(tg, a.in_bstride);
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      T v0, v1;
-      load_pair(src + dep_k[k], v0, v1);
-      const int e = 2 * tid + 2 * kThreads * k;
-      tile[lds_pos(e)] = v0;
-      tile[lds_pos(e + 1)] = v1;
-    }
-  }
-  const T* ops_b = op + (tg >> a.log2_tiles) * a.op_bstride;
+  const int64_t b = tg >> a.log2_tiles;
+  const int64_t origin = int64_t(insert_zero_bits(
+      uint64_t(tg) & ((uint64_t(1) << a.log2_tiles) - 1), a.local, TB));
+  const T* ops_b = op + b * a.op_bstride;
   for (int st = 0; st < a.num_stages; ++st) {
-    __syncthreads();
     const int sb[4] = {a.stage_bits[st][0], a.stage_bits[st][1], a.stage_bits[st][2],
                        a.stage_bits[st][3]};
     const int e0 = int(insert_zero_bits(uint64_t(tid), sb, 4));
     const int m0 = 1 << sb[0], m1 = 1 << sb[1], m2 = 1 << sb[2], m3 = 1 << sb[3];
+    const bool first = st == 0, last = st == a.num_stages - 1;
+    // the first and the last stage hold tile bit 0 (= state bit 0): their
+    // cubes are 8 pairs of adjacent amplitudes, read from and written to the
+    // state without a trip through LDS
+    int64_t off = 0;
+    int64_t d1 = 0, d2 = 0, d3 = 0;
+    if (first || last) {
+      for (int i = 0; i < TB; ++i) off |= int64_t((e0 >> i) & 1) << a.local[i];
+      d1 = int64_t(1) << a.local[sb[1]];
+      d2 = int64_t(1) << a.local[sb[2]];
+      d3 = int64_t(1) << a.local[sb[3]];
+    }
     T c[kCube];
+    if (first) {
+      const T* src = in + b * a.in_bstride + origin + off;
 #pragma unroll
-    for (int j = 0; j < kCube; ++j) {
-      const int e = e0 | ((j & 1) ? m0 : 0) | ((j & 2) ? m1 : 0) | ((j & 4) ? m2 : 0) |
-                    ((j & 8) ? m3 : 0);
-      c[j] = tile[lds_pos(e)];
+      for (int j = 0; j < kCube; j += 2)
+        load_pair(src + ((j & 2) ? d1 : 0) + ((j & 4) ? d2 : 0) + ((j & 8) ? d3 : 0), c[j],
+                  c[j + 1]);
+    } else {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kCube; ++j) {
+        const int e = e0 | ((j & 1) ? m0 : 0) | ((j & 2) ? m1 : 0) | ((j & 4) ? m2 : 0) |
+                      ((j & 8) ? m3 : 0);
+        c[j] = tile[lds_pos(e)];
+      }
     }
     const int act = a.stage_apply[st];
 #define UA_LAYER_BIT(K)                                                       \
@@ -185,19 +208,20 @@ __global__ __launch_bounds__((1 << TB) / kCube) void allq_pass_kernel(T* out, co
     UA_LAYER_BIT(2)
     UA_LAYER_BIT(3)
 #undef UA_LAYER_BIT
+    if (last) {
+      T* dst = out + b * N + origin + off;
 #pragma unroll
-    for (int j = 0; j < kCube; ++j) {
-      const int e = e0 | ((j & 1) ? m0 : 0) | ((j & 2) ? m1 : 0) | ((j & 4) ? m2 : 0) |
-                    ((j & 8) ? m3 : 0);
-      tile[lds_pos(e)] = c[j];
+      for (int j = 0; j < kCube; j += 2)
+        store_pair(dst + ((j & 2) ? d1 : 0) + ((j & 4) ? d2 : 0) + ((j & 8) ? d3 : 0), c[j],
+                   c[j + 1]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < kCube; ++j) {
+        const int e = e0 | ((j & 1) ? m0 : 0) | ((j & 2) ? m1 : 0) | ((j & 4) ? m2 : 0) |
+                      ((j & 8) ? m3 : 0);
+        tile[lds_pos(e)] = c[j];
+      }
     }
-  }
-  __syncthreads();
-  T* dst = out + origin_of(tg, N);
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    const int e = 2 * tid + 2 * kThreads * k;
-    store_pair(dst + dep_k[k], tile[lds_pos(e)], tile[lds_pos(e + 1)]);
   }
 }
 
@@ -228,19 +252,40 @@ int plan_layer(int n, uint64_t active, const int* slot, int TB, int R, AllqPass*
       local &= local - 1;
       if ((gates >> p.local[i]) & 1) pos_of_gate[ng++] = i;
     }
-    p.num_stages = 0;
-    for (int g0 = 0; g0 < ng; g0 += 4) {
-      const int st = p.num_stages++;
-      int cube[4], nc = 0;
-      for (int g = g0; g < ng && g < g0 + 4; ++g) cube[nc++] = pos_of_gate[g];
-      const int applied = nc;
-      for (int t = 0; nc < 4; ++t) {  // pad with tile bits outside this cube
+    // Stages.  The first and the last move their cubes straight from and to
+    // the state, so both hold tile bit 0 and up to three other gates (high tile
+    // bits, which leaves the low ones to the lanes); the gates in between go
+    // four to a stage.  Gates on at most four bits with bit 0 among the
+    // cube need one stage and no LDS.
+    const bool gate0 = ng > 0 && pos_of_gate[0] == 0;
+    int others[kMaxTileBits], no = 0;  // gates above tile bit 0, descending
+    for (int g = ng - 1; g >= (gate0 ? 1 : 0); --g) others[no++] = pos_of_gate[g];
+    p.num_stages = no <= 3 ? 1 : 2 + (no > 6 ? (no - 6 + 3) / 4 : 0);
+    int taken = 0;
+    for (int st = 0; st < p.num_stages; ++st) {
+      const bool first = st == 0, end = first || st == p.num_stages - 1;
+      int cube[4], on[4], nc = 0;
+      if (end) {
+        cube[nc] = 0;
+        on[nc++] = first && gate0;
+      }
+      // the last stage takes what is left, at most three
+      const int left = no - taken, later = p.num_stages - 1 - st;
+      int take = end ? 3 : 4;
+      if (later == 0) take = left;
+      else if (take > left) take = left;
+      for (int i = 0; i < take; ++i) {
+        cube[nc] = others[taken++];
+        on[nc++] = 1;
+      }
+      for (int t = TB - 1; nc < 4; --t) {  // pad with tile bits outside this cube
         bool used = false;
         for (int c = 0; c < nc; ++c) used |= cube[c] == t;
-        if (!used) cube[nc++] = t;
+        if (!used) {
+          cube[nc] = t;
+          on[nc++] = 0;
+        }
       }
-      int on[4];
-      for (int k = 0; k < 4; ++k) on[k] = k < applied;
       for (int i = 1; i < 4; ++i)  // ascending tile bits (insert_zero_bits needs it)
         for (int j = i; j > 0 && cube[j - 1] > cube[j]; --j) {
           const int c = cube[j]; cube[j] = cube[j - 1]; cube[j - 1] = c;

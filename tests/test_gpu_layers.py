@@ -223,3 +223,23 @@ def test_act_last_qubit(device):
                                  torch.from_numpy(batch).to(device)).cpu().numpy()
     assert rel(out, U.act_last_qubit(op.astype(np.complex128),
                                      batch.astype(np.complex128))) < 2e-6
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("count", [1, 3, 4, 5, 6, 7, 8, 11, 12, 13])
+@pytest.mark.parametrize("with_bit0", [False, True])
+def test_layer_stage_counts(device, dt, count, with_bit0):
+    """Every number of stages of a pass (first and last stages read and write
+    the state directly; bit 0 of the tile with and without a gate)."""
+    n = 14
+    rng = np.random.default_rng(100 + count)
+    qubits = [int(q) for q in rng.permutation(n - 1)[:count - 1 if with_bit0 else count]]
+    if with_bit0:
+        qubits.insert(count // 2, n - 1)
+    ops = [cast(rand((2, 2), dt, rng), dt) for _ in qubits]
+    st = cast(rand((3, 2 ** n), dt, rng), dt)
+    out = sim.apply_to_qubits([torch.from_numpy(o).to(device) for o in ops], qubits,
+                              torch.from_numpy(st).to(device))
+    ref = U.apply_to_qubits([o.astype(np.complex128) for o in ops], qubits,
+                            st.astype(np.complex128))
+    assert rel(out.cpu().numpy(), ref) < TOL[dt] * count
