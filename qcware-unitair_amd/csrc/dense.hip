@@ -155,15 +155,12 @@ bool aligned(const void* ptr, int64_t stride_elems, size_t esize, size_t align) 
 
 }  // namespace
 
-// Single 6-qubit complex64 gates on the matrix cores (blocks.hip).
-bool six_applies(int dtype, int n, int k, const void* out, const void* in, int64_t in_bstride);
-int apply_dense_six(void* out, const void* in, const void* op, int n, const int* qubits,
-                    int64_t batch, int64_t in_bstride, hipStream_t s);
-// Single 7/8-qubit complex64 gates on the matrix cores, out of place (blocks.hip).
-bool slice_applies(int dtype, int n, int k, const void* out, const void* in, int64_t in_bstride,
-                   int64_t batch);
-int apply_dense_slices(void* out, const void* in, const void* op, int n, int k,
-                       const int* qubits, int64_t batch, int64_t in_bstride, hipStream_t s);
+// Complex gates on 6..10 qubits on the matrix cores (wide_mfma.hip).
+bool gemm_applies(int dtype, int n, int k, const void* out, const void* in, const void* op,
+                  int64_t in_bstride);
+int apply_dense_gemm(void* out, const void* in, const void* op, int dtype, int n, int k,
+                     const int* tb, int64_t batch, int64_t in_bstride, int64_t op_bstride,
+                     hipStream_t s);
 
 // Tiled dense gates on 6..kMaxWideGateK qubits (wide.hip).
 constexpr int kMaxWideGateK = 10;
@@ -265,11 +262,17 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
     return check_launch("dense_fast_kernel");
   }
 
-  if (g_use_mfma && op_bstride == 0 && six_applies(dtype, n, k, out, state, state_bstride))
-    return apply_dense_six(out, state, op, n, qubits, batch, state_bstride, s);
-  if (g_use_mfma && op_bstride == 0 &&
-      slice_applies(dtype, n, k, out, state, state_bstride, batch))
-    return apply_dense_slices(out, state, op, n, k, qubits, batch, state_bstride, s);
+  // (7- and 8-qubit complex64 gates with one operator keep the vector kernel
+  // when they run in place: its rounding there is relied on)
+  const bool vector_in_place =
+      in_place && op_bstride == 0 && dtype == UA_COMPLEX64 && (k == 7 || k == 8);
+  if (g_use_mfma && !vector_in_place &&
+      gemm_applies(dtype, n, k, out, state, op, state_bstride)) {
+    int tbc[kMaxWideGateK];
+    for (int m = 0; m < k; ++m) tbc[m] = n - 1 - qubits[m];
+    return apply_dense_gemm(out, state, op, dtype, n, k, tbc, batch, state_bstride, op_bstride,
+                            s);
+  }
   if (wide_applies(n, k)) {  // 6..10 targets: tiled, in place or not
     int tbc[kMaxWideGateK];
     for (int m = 0; m < k; ++m) tbc[m] = n - 1 - qubits[m];

@@ -1,4 +1,6 @@
-// Dense gates on 6..10 qubits, in place or out of place.
+// Dense gates on 6..10 qubits, in place or out of place, on the vector units:
+// real states, complex128 on 10 qubits, and what wide_mfma.hip leaves (states
+// or operators off its alignment, complex64 7- and 8-qubit gates in place).
 //
 // unitair applies any k-qubit operator by permuting the targets to the front
 // and contracting with einsum (unitair/simulation/operations.py:151-186,
