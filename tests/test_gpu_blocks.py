@@ -131,3 +131,42 @@ def test_blocks_misaligned_state_runs_gate_by_gate(device):
     fe, ma = BAR[torch.complex64]
     got = view.cpu().numpy()
     assert U.fidelity_error(ref, got) < fe and U.max_abs_error(ref, got) < ma
+
+
+# where a pass's first and last gates meet the state: targets on index bits 0
+# and 1 or off them, one to three gates, 4- and 5-qubit ones; 4 tiles (no order
+# of tiles), 8 (one XCD's group each) and 256 (groups of 32)
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n,batch", [(14, 1), (14, 3), (15, 1), (20, 1)])
+@pytest.mark.parametrize("bits", [[(0, 1, 2, 3, 4)], [(2, 3, 4, 5)], [(5, 2, 9, 3, 11)],
+                                  [(1, 7, 4, 10), (8, 2, 3, 9, 5)],
+                                  [(9, 2, 3, 4, 5), (0, 6, 7, 8)],
+                                  [(5, 3, 2, 4), (2, 6, 3, 7, 4), (7, 0, 1, 5)]])
+def test_blocks_first_and_last_gates(device, dt, n, batch, bits):
+    rng = np.random.default_rng(17 * n + len(bits))
+    gates = [Gate("dense", tuple(n - 1 - b for b in bs), matrix=haar_unitary(2 ** len(bs), rng))
+             for bs in bits] * 2         # an odd pass walks the tiles backwards
+    circ = Circuit(n, gates)
+    psi = seeded_state_np(n, (batch,), seed=n)
+    ref = np.stack([oc.run_closed_form(circ.gates, p) for p in psi])
+    got, _ = run_blocks(circ, psi, dt, device)
+    fe, ma = BAR[dt]
+    assert np.max(U.fidelity_error(ref, got)) < fe and U.max_abs_error(ref, got) < ma
+
+
+def test_blocks_misaligned_matrix_runs_gate_by_gate(device):
+    """Matrices that start 8 bytes past a 16-byte boundary: same result."""
+    n = 14
+    circ = fused_dense_circuit(seed=3, n=n, n5=3, n4=2)
+    psi = seeded_state_np(n, (), seed=4)
+    runner = CircuitRunner(circ, dtype=torch.complex64, device=device, dense_blocks=True)
+    pool = runner._buffers[0]
+    shifted = torch.zeros(pool.numel() + 1, dtype=pool.dtype, device=device)
+    shifted[1:].copy_(pool)
+    for i in range(len(circ.gates)):
+        runner._gates[i].data += shifted.data_ptr() + 8 - pool.data_ptr()
+    x = torch.from_numpy(psi).to(device, torch.complex64)
+    got = runner.run(x).cpu().numpy()
+    ref = oc.run_closed_form(circ.gates, psi)
+    fe, ma = BAR[torch.complex64]
+    assert U.fidelity_error(ref, got) < fe and U.max_abs_error(ref, got) < ma
