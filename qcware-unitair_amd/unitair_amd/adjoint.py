@@ -16,9 +16,13 @@ states: psi, and the co-state lam = H psi carried back through the inverse
 gates.  For U(t) = exp(-i t P) the derivative of <psi|H|psi> is
 2 Im <lam|P|psi> at the point right after the gate.  Rotations on distinct
 qubits commute, so a run of them ("group") shares one (lam, psi) point, and
-one ua_pauli_gradients call per Pauli kind gives every qubit's value.  psi
-and lam are stored as one (2B, 2^n) batch, so every inverse step is one fused
-pass over both.  Un-applying gates in complex64 drifts, so psi is
+one ua_pauli_gradients call per Pauli kind gives every qubit's value.  A group
+of z rotations can be evaluated past its own inverse and past the CZs before
+it, because Z commutes with them: it then shares the point of the group before,
+and its inverse is part of that step (one pass over the states and one read of
+them less for each layer of a z-y ansatz).  CZs after the last rotation commute
+with the observable and are left out.  psi and lam are stored as one (2B, 2^n)
+batch, so every inverse step is one fused program over both.  Un-applying gates in complex64 drifts, so psi is
 re-synchronised from checkpoints taken every ceil(sqrt(groups)) groups.
 Memory: two states plus ceil(sqrt(groups)) checkpoints.
 """
@@ -84,6 +88,9 @@ class _Spec:
             fixed = []
         self.segments = segments
         self.trailing = fixed
+        # what the loss and its gradient need of them: CZs are diagonal with
+        # entries of modulus 1, so neither changes with them
+        self.trailing_seen = [] if all(it.kind == "cz" for it in fixed) else fixed
 
     def _fixed_item(self, g):
         n = self.n
@@ -127,7 +134,7 @@ def _rotation_table(spec, params, dtype, sign, repeat=1):
         dev = params.device
         ckey = (spec.key, kind, sign, params.dtype, str(dev))
         consts = _GROUP_INDEX.get(ckey) if spec.key is not None else None
-        if consts is None:       # device constants, made once per gate list (see _group_index)
+        if consts is None:       # device constants, made once per gate list (see _value_blocks)
             consts = (torch.tensor(idxs, device=dev),
                       torch.tensor(coefs, dtype=params.dtype, device=dev))
             if spec.key is not None:
@@ -176,18 +183,22 @@ def _gates_key(gates, n: int, num_params: int) -> int:
 _GROUP_INDEX = {}
 
 
-def _group_index(spec, s, rot, dev):
-    """Device index tensors of rotation group s (Pauli kind, qubit,
-    parameter index, 2 * coefficient), made once per gate list and device:
-    building them per call would copy from the host, which waits for the
-    stream, once per group."""
-    key = (spec.key, s, str(dev))
+def _value_blocks(spec, dev):
+    """{(segment, Pauli kind): block of values} and, for every rotation, device
+    index tensors (block, qubit, parameter index, 2 * coefficient), made once
+    per gate list and device: building them per call would copy from the host,
+    which waits for the stream."""
+    key = (spec.key, "blocks", str(dev))
     hit = _GROUP_INDEX.get(key) if spec.key is not None else None
     if hit is None:
-        hit = (torch.tensor([_PAULI[r[0]] for r in rot], device=dev),
-               torch.tensor([r[1] for r in rot], device=dev),
-               torch.tensor([r[2] for r in rot], device=dev),
-               torch.tensor([2.0 * r[3] for r in rot], dtype=torch.float64, device=dev))
+        blocks, rows = {}, []
+        for s, (_, rot) in enumerate(spec.segments):
+            for kind, q, idx, coef in rot:
+                blk = blocks.setdefault((s, kind), len(blocks))
+                rows.append((blk, q, idx, 2.0 * coef))
+        cols = list(zip(*rows)) if rows else [(), (), (), ()]
+        hit = (blocks, tuple(torch.tensor(c, dtype=torch.int64, device=dev) for c in cols[:3]) +
+               (torch.tensor(cols[3], dtype=torch.float64, device=dev),))
         if spec.key is not None:
             if len(_GROUP_INDEX) >= 4 * _TEMPLATE_LIMIT:
                 _GROUP_INDEX.pop(next(iter(_GROUP_INDEX)))
@@ -246,19 +257,76 @@ class _Programs:
                 items += list(fixed) + _rot_items(s, rot, fwd_table, n)
             self.fwd.append((c0, _program(items, n, dtype, dev, spec.compiled,
                                           (spec.key, "fwd", c0))))
-        self.trail = _program(list(spec.trailing), n, dtype, dev, spec.compiled,
+        self.trail = _program(list(spec.trailing_seen), n, dtype, dev, spec.compiled,
                               (spec.key, "trail"))
-        self.inv_trail = self.inv = None
+        self.back = None
         if backward:
-            inv_table = _rotation_table(spec, p, dtype, -1.0, repeat=2)
-            self.inv_trail = _program([_inverse_fixed(it) for it in reversed(spec.trailing)],
-                                      n, dtype, dev, spec.compiled, (spec.key, "inv_trail"))
-            self.inv = []
-            for s, (fixed, rot) in enumerate(spec.segments):
-                items = _rot_items(s, rot, inv_table, n)
-                items += [_inverse_fixed(it) for it in reversed(fixed)]
-                self.inv.append(_program(items, n, dtype, dev, spec.compiled,
-                                         (spec.key, "inv", s)))
+            self.back = _backward_steps(spec, _rotation_table(spec, p, dtype, -1.0, repeat=2),
+                                        self.every, dtype, dev)
+
+
+def _backward_steps(spec, table, every, dtype, dev):
+    """The backward pass as a list of steps: ("run", program), ("restore", s)
+    (psi before segment s from its checkpoint) and ("eval", segments) (the
+    gradients of those segments' rotations at this point).  The inverse of the
+    first segment is never needed."""
+    n = spec.n
+    steps, pending = [], []
+    items = [_inverse_fixed(it) for it in reversed(spec.trailing_seen)]
+    last = {}            # qubit -> position in items of a rotation nothing has followed yet
+    merged = []          # (position, table key of the later z rotation)
+
+    def flush():
+        prog = None
+        if items:
+            _merge_z(items, merged, table)
+            prog = _program(list(items), n, dtype, dev, spec.compiled,
+                            (spec.key, "back", len(steps)))
+        if prog is not None:
+            steps.append(("run", prog))
+        items.clear()
+        last.clear()
+        merged.clear()
+
+    for s in range(len(spec.segments) - 1, -1, -1):
+        fixed, rot = spec.segments[s]
+        # z rotations behind CZs only: evaluated at the next group's point
+        defer = s > 0 and all(r[0] == "z" for r in rot) and all(it.kind == "cz" for it in fixed)
+        pending.append(s)
+        if not defer:
+            flush()
+            steps.append(("eval", tuple(pending)))
+            pending = []
+        if s == 0:
+            break
+        for r, (it, q) in enumerate(zip(_rot_items(s, rot, table, n), (x[1] for x in rot))):
+            j = last.get(q)
+            if it.kind == "diag1" and j is not None:
+                merged.append((j, (s, r)))     # one 2x2 matrix: the z rotation times the other
+                del last[q]
+                continue
+            if it.kind == "dense1":
+                last[q] = len(items)
+            items.append(it)
+        if fixed:
+            last.clear()
+        items += [_inverse_fixed(it) for it in reversed(fixed)]
+        if s % every == 0:
+            flush()
+            steps.append(("restore", s))
+    return steps
+
+
+def _merge_z(items, merged, table):
+    """items[j] <- diag(table[key]) @ items[j] for every (j, key), state by
+    state, with a few batched ops."""
+    if not merged:
+        return
+    m = torch.stack([items[j].data for j, _ in merged])               # (R, B, 2, 2)
+    d = torch.stack([table[key] for _, key in merged])                # (R, B, 2)
+    prod = (d.unsqueeze(-1) * m).contiguous()
+    for i, (j, _) in enumerate(merged):
+        items[j] = _Item("dense1", items[j].bits, prod[i], True)
 
 
 # Algorithmic HBM bytes of the last forward and backward (state passes, copies,
@@ -339,29 +407,34 @@ class _AdjointExpectation(torch.autograd.Function):
                                        _lib.stream_handle(dev))
             _lib.check(rc, "apply_diagonal")
             del psi
-            if progs.inv_trail is not None:
-                _run_counted(progs.inv_trail, X, "backward_bytes")
             ws = torch.empty(lib.ua_pauli_gradients_workspace(n, B), dtype=torch.uint8,
                              device=dev)
-            vals = torch.empty(len(_PAULI), B, n, dtype=torch.float64, device=dev)
+            # one (B, n) block of values per (segment, Pauli kind), gathered once at
+            # the end: grad[:, idx] += 2 coef vals[block, :, qubit]
+            blocks, index = _value_blocks(spec, dev)
+            vals = torch.empty(max(1, len(blocks)), B, n, dtype=torch.float64, device=dev)
+            for step, what in progs.back:
+                if step == "run":
+                    _run_counted(what, X, "backward_bytes")
+                elif step == "restore":
+                    X[:B].copy_(ckpt[what])      # psi before that segment, as the forward had it
+                    last_traffic["backward_bytes"] += 2 * _bytes(ckpt[what])
+                else:
+                    for kind in _PAULI:
+                        for s in what:
+                            blk = blocks.get((s, kind))
+                            if blk is None:
+                                continue
+                            rc = lib.ua_pauli_gradients(
+                                _lib.ptr(vals[blk]), _lib.ptr(X[B:]), _lib.ptr(X[:B]),
+                                code[dtype], n, B, _PAULI[kind], _lib.ptr(ws),
+                                _lib.stream_handle(dev))
+                            _lib.check(rc, "pauli_gradients")
+                            last_traffic["backward_bytes"] += _bytes(X)
             grad = torch.zeros(B, params.shape[1], dtype=torch.float64, device=dev)
-            for s in range(len(spec.segments) - 1, -1, -1):
-                fixed, rot = spec.segments[s]
-                for kind in sorted({r[0] for r in rot}):
-                    out = vals[_PAULI[kind]]
-                    rc = lib.ua_pauli_gradients(_lib.ptr(out), _lib.ptr(X[B:]), _lib.ptr(X[:B]),
-                                                code[dtype], n, B, _PAULI[kind], _lib.ptr(ws),
-                                                _lib.stream_handle(dev))
-                    _lib.check(rc, "pauli_gradients")
-                    last_traffic["backward_bytes"] += _bytes(X)
-                # one gather-add per group: grad[:, idx] += 2 coef vals[kind, :, q]
-                kinds, qs, idx, coef = _group_index(spec, s, rot, dev)
-                grad.index_add_(1, idx, vals[kinds, :, qs].transpose(0, 1) * coef)
-                if progs.inv[s] is not None:
-                    _run_counted(progs.inv[s], X, "backward_bytes")
-                if s in ckpt:
-                    X[:B].copy_(ckpt[s])         # psi before segment s, as the forward had it
-                    last_traffic["backward_bytes"] += 2 * _bytes(ckpt[s])
+            if blocks:
+                blk, qs, idx, coef = index
+                grad.index_add_(1, idx, vals[blk, :, qs].transpose(0, 1) * coef)
             grad_p = (grad * gloss.to(torch.float64).view(B, 1)).to(params.dtype)
         return grad_p, grad_obs, None, None, None
 

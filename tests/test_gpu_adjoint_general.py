@@ -158,3 +158,37 @@ def test_general_adjoint_compiled_passes(device, n, dtype):
             assert abs(g[0, i] - ps) < 1e-9, i
     loss2, g2, _ = _run(device, params, gates, obs, n, dtype, compiled=True)
     assert np.array_equal(loss2, loss) and np.array_equal(g2, g)
+
+
+def _layers(pattern, n):
+    """Gates from a pattern of letters: z/y/x: that rotation on every qubit (parameter
+    of its own); c: a CZ ring; n: a CNOT; w: z rotations on every other qubit."""
+    gates, p = [], 0
+    for ch in pattern:
+        if ch == "c":
+            gates += [("cz", q, (q + 1) % n) for q in range(n)]
+        elif ch == "n":
+            gates.append(("cnot", 1, 3))
+        else:
+            for q in range(0, n, 2 if ch == "w" else 1):
+                gates.append(("z" if ch == "w" else ch, q, p, 0.5 + 0.1 * q))
+                p += 1
+    return gates, p
+
+
+@pytest.mark.parametrize("pattern", ["zyczyc", "yzczwcy", "zzyz", "czyczyczyczyc", "ywxcwnzc",
+                                     "zczn", "ynzcyczn", "z", "xzyxzcczyx"])
+def test_z_groups_share_the_point_of_the_group_before(device, pattern):
+    """z groups behind CZs are evaluated past their inverse: first, last, in
+    runs, partial, behind a CNOT (not shared), across the checkpoints of longer
+    lists, and CZs (left out) or a CNOT after the last rotation."""
+    n, B = 5, 2
+    gates, P = _layers(pattern, n)
+    rng = np.random.default_rng(len(pattern))
+    params = rng.uniform(-np.pi, np.pi, (B, P))
+    obs = rng.standard_normal(2 ** n)
+    loss, g, _ = _run(device, params, gates, obs, n, torch.complex128)
+    for b in range(B):
+        assert abs(loss[b] - AO.general_loss(params[b], gates, obs, n)) < 1e-11
+        for i in range(P):
+            assert abs(g[b, i] - AO.general_param_shift(params[b], gates, obs, n, i)) < 1e-10
