@@ -512,8 +512,10 @@ int ua_operator_gradient(void* grad_op, const void* grad_out, const void* state,
  *                   angle t of a rotation exp(-i t/2 P_q) sitting where (lambda,
  *                   psi) were taken (twice that for unitair's exp_x/exp_y/exp_z(t)
  *                   = exp(-i t P), gates.py:7-91).
- * Workspace: ua_pauli_gradients_workspace(num_qubits, batch) bytes (both
- * ua_expect_sum_z and ua_pauli_gradients).  complex64/complex128 states.
+ * ua_pauli_gradients_z  the X or Y gradients, and the Z gradients at the same
+ *                   point in z_out, with one read of both states less.
+ * Workspace: ua_pauli_gradients_workspace(num_qubits, batch) bytes (for
+ * ua_expect_sum_z and both gradient entry points).  complex64/complex128 states.
  */
 enum { UA_PAULI_X = 0, UA_PAULI_Y = 1, UA_PAULI_Z = 2 };
 int64_t ua_pauli_gradients_workspace(int num_qubits, int64_t batch);
@@ -524,6 +526,9 @@ int ua_apply_sum_z(void* out, const void* psi, int dtype, int num_qubits, int64_
 int ua_pauli_gradients(double* out, const void* lambda, const void* psi, int dtype,
                        int num_qubits, int64_t batch, int pauli, void* workspace,
                        ua_stream_t stream);
+int ua_pauli_gradients_z(double* out, double* z_out, const void* lambda, const void* psi,
+                         int dtype, int num_qubits, int64_t batch, int pauli, void* workspace,
+                         ua_stream_t stream);
 
 /* ua_apply_diagonal  out = d * psi elementwise for a real diagonal d (float32
  *                    or float64; diag_batch_stride 0 = one row for every state,

@@ -41,6 +41,28 @@ __device__ __forceinline__ double wave_sum(double v) {
   return v;
 }
 
+// Sums of 16 values over a wavefront at once: at each of the first four steps a
+// lane hands half of its values to its partner and keeps the sums of the other
+// half, the last two steps add what is left (17 exchanges; 16 sums one after
+// another take 96).  Returns the sum of value `which`, the lane's top four bits.
+__device__ __forceinline__ double wave_sums(double (&v)[16], int& which) {
+  const int lane = threadIdx.x & 63;
+  int cnt = 16;
+  which = 0;
+#pragma unroll
+  for (int m = 32; m >= 4; m >>= 1) {
+    cnt >>= 1;
+    const bool upper = lane & m;
+#pragma unroll
+    for (int i = 0; i < cnt; ++i)
+      v[i] = (upper ? v[i + cnt] : v[i]) + __shfl_xor(upper ? v[i] : v[i + cnt], m, 64);
+    which += upper ? cnt : 0;
+  }
+  v[0] += __shfl_xor(v[0], 2, 64);
+  v[0] += __shfl_xor(v[0], 1, 64);
+  return v[0];
+}
+
 // Sums v over the workgroup (256 threads); result in thread 0.
 __device__ double block_sum(double v, double* scratch) {
   v = wave_sum(v);
@@ -118,24 +140,25 @@ __device__ __forceinline__ double pair_term_of(double2 l0, double2 l1, double2 p
   return pair_term<P>(l0, l1, p0, p1);
 }
 
-// The same sums for a full 4096-amplitude tile (m = 12, every state of 12 or
-// more qubits) with the work in registers: after a coalesced copy of both
-// tiles into LDS, each thread reads three 16-amplitude cubes (tile bits 0..3,
-// 4..7, 8..11) and adds the pair terms of the cube's 4 bits; the 12 sums stay
-// in registers until one reduction at the end.  LDS position of element e:
-// e ^ ((e >> 4) & 15), so the copy and all three cube reads touch distinct
-// banks across 16 lanes.
+// The same sums for full 4096-amplitude tiles (m = 12, every state of 12 or more
+// qubits) with the work in registers: a thread's 16 loads of either state are the
+// cube of tile bits 8..11; both tiles go to LDS, from where it reads the cubes of
+// bits 0..3 and 4..7, and it adds the pair terms of each cube's 4 bits.  The sums
+// stay in registers over all tiles of the workgroup until one reduction.  LDS
+// position of element e: e ^ ((e >> 4) & 15), so the copy and both cube reads
+// touch distinct banks across 16 lanes.
+//
+// 16 qubits x 1024 states, complex64 (1 GiB of both states): 262 us with Z, where
+// X / Y took 295 and Z another 264.  What it cost was the reduction, 12 sums of
+// every wavefront for each tile; one for a run of tiles and 17 exchanges for 16
+// sums leave the reads (4.1 TB/s) and LDS.  More wavefronts with smaller cubes
+// were slower (504 us), the next tile's loads ahead too (385, spilled registers).
 __device__ __forceinline__ int low_swz(int e) { return e ^ ((e >> 4) & 15); }
 
+constexpr int kMaxRun = 16;  // tiles of a workgroup
+
 template <int P, int B0, typename T>
-__device__ __forceinline__ void low_cube(double (&acc)[kLowBits], const T* sl, const T* sp,
-                                         int e0) {
-  T l[16], p[16];
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    l[j] = sl[low_swz(e0 | (j << B0))];
-    p[j] = sp[low_swz(e0 | (j << B0))];
-  }
+__device__ __forceinline__ void cube_terms(double (&acc)[16], const T (&l)[16], const T (&p)[16]) {
 #pragma unroll
   for (int k = 0; k < 4; ++k)
 #pragma unroll
@@ -146,103 +169,179 @@ __device__ __forceinline__ void low_cube(double (&acc)[kLowBits], const T* sl, c
     }
 }
 
-// complex64 tiles (64 KiB of LDS) leave room for two workgroups per CU:
-// the register budget asks for both
-template <typename T>
-constexpr int low_full_waves() { return sizeof(T) == 8 ? 2 : 1; }
+template <int P, int B0, typename T>
+__device__ __forceinline__ void low_cube(double (&acc)[16], const T* sl, const T* sp, int e0) {
+  T l[16], p[16];
+#pragma unroll
+  for (int j = 0; j < 16; ++j) {
+    l[j] = sl[low_swz(e0 | (j << B0))];
+    p[j] = sp[low_swz(e0 | (j << B0))];
+  }
+  cube_terms<P, B0>(acc, l, p);
+}
 
-template <typename T, int P>
+// A workgroup takes `run` (a power of two, at most 16) consecutive tiles of a
+// state: partial[(b * runs + r) * n + bit].
+// Z: also the Z gradients, in zpartial[(b * runs + r) * n + qubit].  The thread
+// that copies elements tid + 256 k has the cube of bits 8..11 in registers, so
+// those bits and Z need no read of LDS.
+template <typename T, int P, bool Z>
 __global__ __launch_bounds__(kBlock)
-__attribute__((amdgpu_waves_per_eu(low_full_waves<T>()))) void grad_low_full_kernel(
-    double* __restrict__ partial, const T* __restrict__ lam, const T* __restrict__ psi, int n,
-    int64_t tiles_per_state) {
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 2 : 1))) void grad_low_full_kernel(
+    double* __restrict__ partial, double* __restrict__ zpartial, const T* __restrict__ lam,
+    const T* __restrict__ psi, int n, int64_t runs_per_state, int run) {
   __shared__ T sl[kLowTile];
   __shared__ T sp[kLowTile];
-  __shared__ double red[kBlock / 64][kLowBits];
-  const int64_t tile = blockIdx.x;
-  const int64_t b = tile / tiles_per_state;
-  const int64_t t = tile % tiles_per_state;
+  __shared__ double red[kBlock / 64][16];
+  __shared__ double zred[kBlock / 64][16];
+  const int64_t b = blockIdx.x / runs_per_state;
+  const int64_t r0 = blockIdx.x % runs_per_state;
   const int64_t N = int64_t(1) << n;
   const int tid = threadIdx.x;
-  const T* L = lam + b * N + t * kLowTile;
-  const T* Ps = psi + b * N + t * kLowTile;
-#pragma unroll
-  for (int k = 0; k < kLowTile / kBlock; ++k) {
-    const int i = tid + k * kBlock;
-    sl[low_swz(i)] = L[i];
-    sp[low_swz(i)] = Ps[i];
-  }
-  __syncthreads();
-  double acc[kLowBits];
-#pragma unroll
-  for (int i = 0; i < kLowBits; ++i) acc[i] = 0.0;
-  // thread tid's cube entry 0: tid's 8 bits around the cube's 4
-  // (the empty asm keeps each cube's LDS reads after the previous cube's
-  // arithmetic: with all three cubes' reads hoisted the registers overflow)
-  low_cube<P, 0>(acc, sl, sp, tid << 4);
-  asm volatile("" ::: "memory");
-  low_cube<P, 4>(acc, sl, sp, (tid & 15) | ((tid >> 4) << 8));
-  asm volatile("" ::: "memory");
-  low_cube<P, 8>(acc, sl, sp, tid);
   const int lane = tid & 63, wave = tid >> 6;
+  const T* L = lam + b * N + r0 * run * kLowTile + tid;
+  const T* Ps = psi + b * N + r0 * run * kLowTile + tid;
+  double acc[16];
+  // signed sums of Z: bits 8..11 (0..3), bits 12..15 within the run (4..7), the total (8)
+  double z[Z ? 9 : 1];
 #pragma unroll
-  for (int i = 0; i < kLowBits; ++i) {
-    const double v = wave_sum(acc[i]);
-    if (lane == 0) red[wave][i] = v;
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0;
+#pragma unroll
+  for (int i = 0; i < (Z ? 9 : 1); ++i) z[i] = 0.0;
+  for (int t = 0; t < run; ++t, L += kLowTile, Ps += kLowTile) {
+    T l[16], p[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      l[k] = L[k * kBlock];
+      p[k] = Ps[k * kBlock];
+    }
+    if (t > 0) __syncthreads();  // the tile before is read
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      sl[low_swz(tid + k * kBlock)] = l[k];
+      sp[low_swz(tid + k * kBlock)] = p[k];
+    }
+    __syncthreads();
+    cube_terms<P, 8>(acc, l, p);
+    if constexpr (Z) {
+      double total = 0.0;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const double v = im_cj(D2<T>::get(l[k]), D2<T>::get(p[k]));
+        total += v;
+#pragma unroll
+        for (int bit = 0; bit < 4; ++bit) z[bit] += ((k >> bit) & 1) ? -v : v;
+      }
+#pragma unroll
+      for (int bit = 0; bit < 4; ++bit) z[4 + bit] += ((t >> bit) & 1) ? -total : total;
+      z[8] += total;
+    }
+    // the empty asm keeps the LDS reads of each part after the arithmetic of the
+    // one before: all hoisted, the registers overflow
+    asm volatile("" ::: "memory");
+    // thread tid's cube entry 0: tid's 8 bits around the cube's 4
+    low_cube<P, 0>(acc, sl, sp, tid << 4);
+    asm volatile("" ::: "memory");
+    low_cube<P, 4>(acc, sl, sp, (tid & 15) | ((tid >> 4) << 8));
+  }
+  int which;
+  const double sum = wave_sums(acc, which);
+  if ((lane & 3) == 0) red[wave][which] = sum;
+  if constexpr (Z) {
+    double v[16];  // z as it is, then bits 0..5 as 9..14
+#pragma unroll
+    for (int i = 0; i < 9; ++i) v[i] = z[i];
+#pragma unroll
+    for (int bit = 0; bit < 6; ++bit) v[9 + bit] = ((tid >> bit) & 1) ? -z[8] : z[8];
+    v[15] = 0.0;
+    const double zs = wave_sums(v, which);
+    if ((lane & 3) == 0) zred[wave][which] = zs;
   }
   __syncthreads();
   if (tid < kLowBits) {
     double r = 0.0;
 #pragma unroll
     for (int w = 0; w < kBlock / 64; ++w) r += red[w][tid];
-    partial[(b * tiles_per_state + t) * n + tid] = r;
+    partial[(b * runs_per_state + r0) * n + tid] = r;
+  }
+  if constexpr (Z) {
+    if (tid < n) {
+      const int bit = tid;  // index bit: of the lanes, the wavefronts, the cube, the run or above
+      const bool in_run = bit >= kLowBits && bit < kLowBits + 4 && (run >> (bit - kLowBits)) > 1;
+      double r = 0.0;
+#pragma unroll
+      for (int w = 0; w < kBlock / 64; ++w) {
+        const double total = zred[w][8];
+        if (bit < 6) r += zred[w][9 + bit];
+        else if (bit < 8) r += ((w >> (bit - 6)) & 1) ? -total : total;
+        else if (bit < kLowBits) r += zred[w][bit - 8];
+        else if (in_run) r += zred[w][4 + bit - kLowBits];
+        else r += (((r0 * run) >> (bit - kLowBits)) & 1) ? -total : total;
+      }
+      zpartial[(b * runs_per_state + r0) * n + (n - 1 - bit)] = r;
+    }
   }
 }
 
 // X / Y gradients for a window of H index bits w0..w0+H-1 (w0 >= 12).  Each
 // thread owns one low index (bits 0..11: 256 consecutive per workgroup, so
 // every load is coalesced) and, for each value r of the other high bits in
-// its block's range, the 2^H amplitudes over the window.
-// partial[((b * 16 + blockIdx.y) * gridDim.z + blockIdx.z) * n + bit].
+// its block's range, the 2^H amplitudes over the window.  A workgroup takes
+// `chunks` neighbouring chunks of 256 low indices, so that one reduction serves
+// them all (16 qubits x 1024 states: 238 -> 214 us, 5.0 TB/s).
+// partial[((b * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z) * n + bit].
 template <typename T, int P, int H>
 __global__ __launch_bounds__(kBlock) void grad_high_kernel(
     double* __restrict__ partial, const T* __restrict__ lam, const T* __restrict__ psi, int n,
-    int w0, int64_t rest_per_block) {
-  __shared__ double scratch[kBlock / 64];
+    int w0, int64_t rest_per_block, int chunks) {
+  __shared__ double red[kBlock / 64][16];
   constexpr int HN = 1 << H;
   const int64_t b = blockIdx.x;
-  const int low = blockIdx.y * kBlock + threadIdx.x;  // < 4096
   const int64_t N = int64_t(1) << n;
   const int below = w0 - kLowBits;                    // other high bits under the window
-  double acc[H];
+  double acc[16];
 #pragma unroll
-  for (int hb = 0; hb < H; ++hb) acc[hb] = 0.0;
+  for (int hb = 0; hb < 16; ++hb) acc[hb] = 0.0;
   const int64_t r0 = int64_t(blockIdx.z) * rest_per_block;
   for (int64_t r = r0; r < r0 + rest_per_block; ++r) {
     const uint64_t rest = ((uint64_t(r) & ((uint64_t(1) << below) - 1)) << kLowBits) |
                           ((uint64_t(r) >> below) << (w0 + H));
-    const int64_t base = b * N + int64_t(rest) + low;
-    double2 l[HN], p[HN];
-#pragma unroll
-    for (int h = 0; h < HN; ++h) {
-      l[h] = D2<T>::get(lam[base + (int64_t(h) << w0)]);
-      p[h] = D2<T>::get(psi[base + (int64_t(h) << w0)]);
-    }
-#pragma unroll
-    for (int hb = 0; hb < H; ++hb) {
+    for (int c = 0; c < chunks; ++c) {
+      const int low = (int(blockIdx.y) * chunks + c) * kBlock + threadIdx.x;  // < 4096
+      const int64_t base = b * N + int64_t(rest) + low;
+      T l[HN], p[HN];
 #pragma unroll
       for (int h = 0; h < HN; ++h) {
-        if (h & (1 << hb)) continue;
-        const int h1 = h | (1 << hb);
-        acc[hb] += pair_term<P>(l[h], l[h1], p[h], p[h1]);
+        l[h] = lam[base + (int64_t(h) << w0)];
+        p[h] = psi[base + (int64_t(h) << w0)];
+      }
+#pragma unroll
+      for (int hb = 0; hb < H; ++hb) {
+        // the amplitudes stay in the state's own type: as float64 for all bits at
+        // once they take twice the registers (230, two wavefronts per SIMD)
+#pragma unroll
+        for (int h = 0; h < HN; ++h)
+          asm volatile("" : "+v"(l[h].x), "+v"(l[h].y), "+v"(p[h].x), "+v"(p[h].y));
+#pragma unroll
+        for (int h = 0; h < HN; ++h) {
+          if (h & (1 << hb)) continue;
+          const int h1 = h | (1 << hb);
+          acc[hb] += pair_term<P>(D2<T>::get(l[h]), D2<T>::get(l[h1]), D2<T>::get(p[h]),
+                                  D2<T>::get(p[h1]));
+        }
       }
     }
   }
   const int64_t part = (b * gridDim.y + blockIdx.y) * gridDim.z + blockIdx.z;
+  int which;
+  const double sum = wave_sums(acc, which);
+  if ((threadIdx.x & 3) == 0) red[threadIdx.x >> 6][which] = sum;
+  __syncthreads();
+  if (threadIdx.x < H) {
+    double t = 0.0;
 #pragma unroll
-  for (int hb = 0; hb < H; ++hb) {
-    const double s = block_sum(acc[hb], scratch);
-    if (threadIdx.x == 0) partial[part * n + w0 + hb] = s;
+    for (int w = 0; w < kBlock / 64; ++w) t += red[w][threadIdx.x];
+    partial[part * n + w0 + threadIdx.x] = t;
   }
 }
 
@@ -387,13 +486,16 @@ extern "C" int64_t ua_pauli_gradients_workspace(int num_qubits, int64_t batch) {
   const int64_t z = z_parts(n) * (n + 1);
   if (h > a) a = h;
   if (z > a) a = z;
+  if (n >= kLowBits && 2 * y_low_parts(n) * n > a) a = 2 * y_low_parts(n) * n;  // X / Y and Z
   return (batch < 1 ? 1 : batch) * a * int64_t(sizeof(double));
 }
 
-extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* psi, int dtype,
-                                  int num_qubits, int64_t batch, int pauli, void* workspace,
-                                  ua_stream_t stream) {
-  const int n = num_qubits;
+namespace ua {
+namespace {
+// z_out: NULL, or where the Z gradients go as well (X / Y on at least 12 qubits;
+// their partials follow the others' in the workspace).
+int pauli_gradients(double* out, double* z_out, const void* lambda, const void* psi, int dtype,
+                    int n, int64_t batch, int pauli, void* workspace, ua_stream_t stream) {
   hipStream_t s = static_cast<hipStream_t>(stream);
   UA_CHECK_ARG(dtype == UA_COMPLEX64 || dtype == UA_COMPLEX128, "complex states only");
   UA_CHECK_ARG(n >= 1 && n <= kMaxN, "num_qubits=%d out of range", n);
@@ -426,12 +528,21 @@ extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* p
   const int m = n < kLowBits ? n : kLowBits;
   const int64_t tiles = y_low_parts(n);
   UA_CHECK_ARG(batch * tiles <= 0x7fffffffLL, "grid too large");
-  const unsigned glow = unsigned(batch * tiles);
+  // full tiles: runs of them for a workgroup, as long as 2048 workgroups are left
+  int run = 1;
+  if (m == kLowBits)
+    while (run < kMaxRun && run < tiles && batch * (tiles / (2 * run)) >= 2048) run *= 2;
+  const int64_t runs = tiles / run;
+  const unsigned glow = unsigned(batch * runs);
+  double* const zpart = part + batch * tiles * n;
 #define UA_LOW(TT, PP)                                                                   \
   do {                                                                                   \
-    if (m == kLowBits)                                                                   \
-      grad_low_full_kernel<TT, PP><<<glow, kBlock, 0, s>>>(part, (const TT*)lambda,      \
-                                                           (const TT*)psi, n, tiles);     \
+    if (m == kLowBits && z_out)                                                          \
+      grad_low_full_kernel<TT, PP, true><<<glow, kBlock, 0, s>>>(                        \
+          part, zpart, (const TT*)lambda, (const TT*)psi, n, runs, run);                     \
+    else if (m == kLowBits)                                                              \
+      grad_low_full_kernel<TT, PP, false><<<glow, kBlock, 0, s>>>(                       \
+          part, nullptr, (const TT*)lambda, (const TT*)psi, n, runs, run);                   \
     else                                                                                 \
       grad_low_kernel<TT, PP><<<glow, kBlock, 0, s>>>(part, (const TT*)lambda,           \
                                                       (const TT*)psi, n, m, tiles);       \
@@ -444,8 +555,14 @@ extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* p
 #undef UA_LOW
   int rc = check_launch("grad_low_kernel");
   if (rc) return rc;
+  if (z_out) {  // stored by qubit
+    sum_parts_kernel<<<grid_for(batch * n), kBlock, 0, s>>>(z_out, zpart, batch, runs, n, 0, n, n,
+                                                            0, 0, 1);
+    rc = check_launch("sum_parts_kernel");
+    if (rc) return rc;
+  }
   // bits 0..m-1 -> qubits n-1 .. n-m, one launch
-  sum_parts_kernel<<<grid_for(batch * m), kBlock, 0, s>>>(out, part, batch, tiles, n, 0, m, n,
+  sum_parts_kernel<<<grid_for(batch * m), kBlock, 0, s>>>(out, part, batch, runs, n, 0, m, n,
                                                           n - 1, 0, -1);
   rc = check_launch("sum_parts_kernel");
   if (rc) return rc;
@@ -457,23 +574,26 @@ extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* p
     const int rest_bits = n - kLowBits - H;
     const int64_t zz = rest_bits > 0 ? z : 1;
     const int64_t per_block = (int64_t(1) << (rest_bits > 0 ? rest_bits : 0)) / zz;
-    const dim3 grid = dim3(unsigned(batch), unsigned(kHighParts), unsigned(zz));
+    int chunks = 1;  // of low indices, as long as 2048 workgroups are left
+    while (chunks < kHighParts && batch * zz * (kHighParts / (2 * chunks)) >= 2048) chunks *= 2;
+    const int64_t parts = kHighParts / chunks;
+    const dim3 grid = dim3(unsigned(batch), unsigned(parts), unsigned(zz));
 #define UA_HIGH(HH)                                                                             \
   if (H == HH) {                                                                               \
     if (pauli == UA_PAULI_X) {                                                                 \
       if (c64)                                                                                 \
         grad_high_kernel<float2, UA_PAULI_X, HH><<<grid, kBlock, 0, s>>>(                      \
-            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block);                \
+            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);                \
       else                                                                                     \
         grad_high_kernel<double2, UA_PAULI_X, HH><<<grid, kBlock, 0, s>>>(                     \
-            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block);              \
+            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);              \
     } else {                                                                                   \
       if (c64)                                                                                 \
         grad_high_kernel<float2, UA_PAULI_Y, HH><<<grid, kBlock, 0, s>>>(                      \
-            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block);                \
+            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);                \
       else                                                                                     \
         grad_high_kernel<double2, UA_PAULI_Y, HH><<<grid, kBlock, 0, s>>>(                     \
-            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block);              \
+            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);              \
     }                                                                                          \
   }
     UA_HIGH(1) UA_HIGH(2) UA_HIGH(3) UA_HIGH(4)
@@ -481,12 +601,39 @@ extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* p
     rc = check_launch("grad_high_kernel");
     if (rc) return rc;
     // bits w0..w0+H-1 -> qubits n-1-w0 .. n-w0-H, one launch
-    sum_parts_kernel<<<grid_for(batch * H), kBlock, 0, s>>>(out, part, batch, kHighParts * zz, n,
+    sum_parts_kernel<<<grid_for(batch * H), kBlock, 0, s>>>(out, part, batch, parts * zz, n,
                                                             w0, H, n, n - 1 - w0, 0, -1);
     rc = check_launch("sum_parts_kernel");
     if (rc) return rc;
   }
   return UA_OK;
+}
+
+// whether one launch can give the Z gradients beside the X / Y ones
+bool z_beside(int n) { return n >= kLowBits; }
+}  // namespace
+}  // namespace ua
+
+extern "C" int ua_pauli_gradients(double* out, const void* lambda, const void* psi, int dtype,
+                                  int num_qubits, int64_t batch, int pauli, void* workspace,
+                                  ua_stream_t stream) {
+  return pauli_gradients(out, nullptr, lambda, psi, dtype, num_qubits, batch, pauli, workspace,
+                         stream);
+}
+
+extern "C" int ua_pauli_gradients_z(double* out, double* z_out, const void* lambda,
+                                    const void* psi, int dtype, int num_qubits, int64_t batch,
+                                    int pauli, void* workspace, ua_stream_t stream) {
+  UA_CHECK_ARG(pauli == UA_PAULI_X || pauli == UA_PAULI_Y, "pauli must be X or Y");
+  UA_CHECK_ARG(batch <= 0 || z_out, "NULL pointer");
+  if (num_qubits >= 1 && num_qubits <= kMaxN && !z_beside(num_qubits)) {
+    const int rc = pauli_gradients(z_out, nullptr, lambda, psi, dtype, num_qubits, batch,
+                                   UA_PAULI_Z, workspace, stream);
+    if (rc) return rc;
+    z_out = nullptr;
+  }
+  return pauli_gradients(out, z_out, lambda, psi, dtype, num_qubits, batch, pauli, workspace,
+                         stream);
 }
 
 namespace ua {

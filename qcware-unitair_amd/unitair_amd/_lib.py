@@ -73,6 +73,7 @@ SIGNATURES = {
     "ua_expect_sum_z": (_i32, [_p, _p, _i32, _i32, _i64, _p, _p]),
     "ua_apply_sum_z": (_i32, [_p, _p, _i32, _i32, _i64, _p]),
     "ua_pauli_gradients": (_i32, [_p, _p, _p, _i32, _i32, _i64, _i32, _p, _p]),
+    "ua_pauli_gradients_z": (_i32, [_p, _p, _p, _p, _i32, _i32, _i64, _i32, _p, _p]),
     "ua_apply_diagonal": (_i32, [_p, _p, _i32, _p, _i32, _i64, _i32, _i64, _p]),
     "ua_apply_cz": (_i32, [_p, _i32, _i32, _i32, _i32, _i64, _p]),
     "ua_apply_cnot": (_i32, [_p, _i32, _i32, _i32, _i32, _i64, _p]),

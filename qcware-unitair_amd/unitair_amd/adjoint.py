@@ -420,17 +420,23 @@ class _AdjointExpectation(torch.autograd.Function):
                     X[:B].copy_(ckpt[what])      # psi before that segment, as the forward had it
                     last_traffic["backward_bytes"] += 2 * _bytes(ckpt[what])
                 else:
-                    for kind in _PAULI:
-                        for s in what:
-                            blk = blocks.get((s, kind))
-                            if blk is None:
-                                continue
-                            rc = lib.ua_pauli_gradients(
-                                _lib.ptr(vals[blk]), _lib.ptr(X[B:]), _lib.ptr(X[:B]),
-                                code[dtype], n, B, _PAULI[kind], _lib.ptr(ws),
-                                _lib.stream_handle(dev))
-                            _lib.check(rc, "pauli_gradients")
-                            last_traffic["backward_bytes"] += _bytes(X)
+                    at = [(kind, blocks[(s, kind)]) for s in what for kind in _PAULI
+                          if (s, kind) in blocks]
+                    # the first Z block rides along with the first X or Y one
+                    zs = [blk for kind, blk in at if kind == "z"]
+                    xys = [(kind, blk) for kind, blk in at if kind != "z"]
+                    both = zs.pop(0) if zs and xys else None
+                    for kind, blk in xys + [("z", blk) for blk in zs]:
+                        args = (_lib.ptr(X[B:]), _lib.ptr(X[:B]), code[dtype], n, B,
+                                _PAULI[kind], _lib.ptr(ws), _lib.stream_handle(dev))
+                        if both is not None:
+                            rc = lib.ua_pauli_gradients_z(_lib.ptr(vals[blk]),
+                                                          _lib.ptr(vals[both]), *args)
+                            both = None
+                        else:
+                            rc = lib.ua_pauli_gradients(_lib.ptr(vals[blk]), *args)
+                        _lib.check(rc, "pauli_gradients")
+                        last_traffic["backward_bytes"] += _bytes(X)
             grad = torch.zeros(B, params.shape[1], dtype=torch.float64, device=dev)
             if blocks:
                 blk, qs, idx, coef = index

@@ -192,3 +192,34 @@ def test_z_groups_share_the_point_of_the_group_before(device, pattern):
         assert abs(loss[b] - AO.general_loss(params[b], gates, obs, n)) < 1e-11
         for i in range(P):
             assert abs(g[b, i] - AO.general_param_shift(params[b], gates, obs, n, i)) < 1e-10
+
+
+@pytest.mark.parametrize("dtype,tol", [(torch.complex128, 1e-12), (torch.complex64, 2e-6)])
+@pytest.mark.parametrize("n,B", [(4, 3), (11, 2), (12, 1), (13, 3), (16, 2), (17, 150), (18, 1)])
+def test_pauli_gradients_with_z(device, dtype, tol, n, B):
+    """X / Y and Z gradients in one call against each other's own sums and a
+    float64 reference: below 12 qubits (separate launches), one tile, runs of
+    tiles within a state (batch 150: two workgroups' worth each) and qubits above
+    a run."""
+    from unitair_amd import _lib
+    lib = _lib.load()
+    g = torch.Generator(device=device).manual_seed(n * 100 + B)
+    real = torch.float64 if dtype == torch.complex128 else torch.float32
+    lam, psi = (torch.view_as_complex(torch.randn(B, 2 ** n, 2, generator=g, device=device,
+                                                  dtype=real)) * 2 ** (-n / 2) for _ in range(2))
+    ws = torch.empty(lib.ua_pauli_gradients_workspace(n, B), dtype=torch.uint8, device=device)
+    l2, p2 = lam.to(torch.complex128), psi.to(torch.complex128)
+    for kind in (_lib.UA_PAULI_X, _lib.UA_PAULI_Y):
+        out, z = (torch.empty(B, n, dtype=torch.float64, device=device) for _ in range(2))
+        rc = lib.ua_pauli_gradients_z(_lib.ptr(out), _lib.ptr(z), _lib.ptr(lam), _lib.ptr(psi),
+                                      _lib.DTYPE_CODES[dtype], n, B, kind, _lib.ptr(ws),
+                                      _lib.stream_handle(device))
+        _lib.check(rc, "pauli_gradients_z")
+        for q in range(n):
+            a, b = (t.reshape(B, 2 ** q, 2, -1) for t in (l2, p2))
+            zr = (a[:, :, 0].conj() * b[:, :, 0] - a[:, :, 1].conj() * b[:, :, 1]).imag
+            c = a[:, :, 0].conj() * b[:, :, 1], a[:, :, 1].conj() * b[:, :, 0]
+            pr = (c[0] + c[1]).imag if kind == _lib.UA_PAULI_X else c[1].real - c[0].real
+            # |lambda| and |psi| are about 1: absolute errors
+            assert float((z[:, q] - zr.sum((1, 2))).abs().max()) < tol
+            assert float((out[:, q] - pr.sum((1, 2))).abs().max()) < tol
