@@ -127,6 +127,43 @@ __global__ __launch_bounds__(kBlock) void phase_pair_kernel(
   }
 }
 
+// TILE layout (one row of angles for every row of the state): a thread owns a
+// column (complex128) or two neighbouring ones (16 bytes of output either way),
+// forms their factors once and multiplies kRows rows at a time by them, so
+// neither the angles nor the sincos are repeated for each state of a batch.  TX
+// threads of a workgroup lie along the columns, kBlock / TX along the rows.
+// 16 qubits x 301 states (complex64): 72 -> 57 us, 5.5 TB/s; the loop over single
+// elements took a 64-bit remainder and a sincos for each.
+constexpr int kRows = 4;
+template <typename T, int W> struct alignas(W * sizeof(T)) Cols { T v[W]; };
+
+template <typename TO, typename TS, typename TA, int TX>
+__global__ __launch_bounds__(kBlock) void phase_rows_kernel(
+    TO* out, const TS* state, const TA* __restrict__ angles, int64_t cols, int64_t rows) {
+  constexpr int TY = kBlock / TX, W = 16 / sizeof(TO);
+  const int64_t c = W * (int64_t(blockIdx.x) * TX + threadIdx.x % TX);
+  if (c >= cols) return;
+  const Cols<TA, W> a = *reinterpret_cast<const Cols<TA, W>*>(angles + c);
+  TO ph[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) ph[w] = Widen<TO>::from(phase_of(a.v[w]));
+  const int64_t step = int64_t(gridDim.y) * TY * kRows;
+  for (int64_t r0 = (int64_t(blockIdx.y) * TY + threadIdx.x / TX) * kRows; r0 < rows; r0 += step) {
+    Cols<TS, W> x[kRows];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      if (r0 + u < rows) x[u] = *reinterpret_cast<const Cols<TS, W>*>(state + (r0 + u) * cols + c);
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      if (r0 + u >= rows) continue;
+      Cols<TO, W> y;
+#pragma unroll
+      for (int w = 0; w < W; ++w) y.v[w] = cmul(ph[w], Widen<TO>::from(x[u].v[w]));
+      *reinterpret_cast<Cols<TO, W>*>(out + (r0 + u) * cols + c) = y;
+    }
+  }
+}
+
 template <typename TO, typename TS, typename TA>
 void launch_phase(int mode, void* out, const void* st, const void* an,
                   const PhaseParams& p, hipStream_t s) {
@@ -144,6 +181,23 @@ void launch_phase(int mode, void* out, const void* st, const void* an,
     const int64_t pairs = p.total / 2;
     phase_pair_kernel<TO, TS, TA, 2><<<grid_for(pairs, kBlock * 2), kBlock, 0, s>>>(o, x, a, pairs);
     return;
+  }
+  // Rows that fill the 64 lanes of a row group at least
+  constexpr int W = 16 / sizeof(TO);
+  if (mode == TILE && pair_ok && p.tile % W == 0 && p.tile >= 64 * W) {
+    const int64_t rows = p.total / p.tile, groups = p.tile / W;
+    const int tx = groups >= kBlock ? kBlock : 64, ty = kBlock / tx;
+    const int64_t gx = (groups + tx - 1) / tx;
+    int64_t gy = (rows + ty * kRows - 1) / (ty * kRows);
+    if (gy > 65535) gy = 65535;
+    if (gx <= 0x7fffffffLL) {
+      const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
+      if (tx == kBlock)
+        phase_rows_kernel<TO, TS, TA, kBlock><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
+      else
+        phase_rows_kernel<TO, TS, TA, 64><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
+      return;
+    }
   }
   switch (mode) {
     case CONTIG: phase_kernel<TO, TS, TA, CONTIG><<<g, kBlock, 0, s>>>(o, x, a, p); break;

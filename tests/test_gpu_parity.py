@@ -448,3 +448,24 @@ def test_wide_gate_unitary_roundtrip_24q(device):
     back = sim.apply_operator(u.conj().T.contiguous(), qubits, y)
     assert abs(float(ua.norm_squared(y)) - 1.0) < 1e-5
     assert float((back - psi).abs().max()) < 1e-5
+
+
+@pytest.mark.parametrize("at,dt", [(torch.float32, torch.complex64),
+                                   (torch.float64, torch.complex128),
+                                   (torch.float32, torch.complex128),
+                                   (torch.complex64, torch.complex64),
+                                   (torch.float32, torch.float32)])
+@pytest.mark.parametrize("cols,rows", [(64, 5), (126, 4), (128, 1), (128, 3), (130, 17), (256, 9),
+                                       (512, 4), (1026, 5), (4096, 33)])
+def test_apply_phase_rows(device, at, dt, cols, rows):
+    """One row of angles for a batch of states: rows too short for, just filling
+    and not filling whole workgroups, row counts around the four taken together.
+    The factors are those of one row, rounded once (2^-24 or 2^-53), and each
+    product rounds three more times."""
+    g = torch.Generator(device=device).manual_seed(cols * 7 + rows)
+    a = torch.randn(cols, generator=g, device=device, dtype=at)
+    x = torch.randn(rows, cols, generator=g, device=device, dtype=dt)
+    out = sim.apply_phase(a, x)
+    ref = torch.exp(-1j * a.to(torch.complex128)) * x.to(torch.complex128)
+    eps = 2.0 ** -24 if torch.float32 in (at, dt) or torch.complex64 in (at, dt) else 2.0 ** -53
+    assert float(((out - ref).abs() / ref.abs()).max()) < 16 * eps
