@@ -55,7 +55,9 @@ class StateShapeError(ValueError):
 
 def count_qubits(state: torch.Tensor) -> int:
     """Number of qubits of a vector-layout state (shapes.py:13-27)."""
-    length = state.size()[-1]
+    length = state.shape[-1]
+    if length > 0 and not length & (length - 1):
+        return length.bit_length() - 1
     n = round(math.log2(length))
     if 2 ** n != length:
         raise StateShapeError(data=state, expected_layout=StateLayout.VECTOR)
@@ -64,7 +66,9 @@ def count_qubits(state: torch.Tensor) -> int:
 
 def count_qubits_gate_matrix(gate: torch.Tensor) -> int:
     """k for a gate of size (*batch, 2^k, 2^k) (shapes.py:31-47)."""
-    length = gate.size()[-1]
+    length = gate.shape[-1]
+    if length > 0 and not length & (length - 1):
+        return length.bit_length() - 1
     k = round(math.log2(length))
     if 2 ** k != length:
         raise RuntimeError(f"Gate matrix of size {tuple(gate.size())} does not act on "

@@ -469,3 +469,43 @@ def test_apply_phase_rows(device, at, dt, cols, rows):
     ref = torch.exp(-1j * a.to(torch.complex128)) * x.to(torch.complex128)
     eps = 2.0 ** -24 if torch.float32 in (at, dt) or torch.complex64 in (at, dt) else 2.0 ** -53
     assert float(((out - ref).abs() / ref.abs()).max()) < 16 * eps
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128, torch.float32])
+@pytest.mark.parametrize("ob,sb", [((), ()), ((), (1,)), ((), (3,)), ((), (2, 3)), ((1,), (1,)),
+                                   ((3,), (3,)), ((2, 3), (2, 3)), ((), (0,)), ((3,), ()),
+                                   ((1, 3), (2, 3))])
+def test_direct_and_general_call_paths_agree(device, dt, ob, sb):
+    """Contiguous operators and states go to the library as they are; the same
+    values in strided memory take the general path: same shape, same bits."""
+    n, qubits = 9, [6, 1]
+    g = torch.Generator(device=device).manual_seed(3)
+    op = torch.randn(ob + (4, 4), generator=g, device=device, dtype=dt)
+    st = torch.randn(sb + (2 ** n,), generator=g, device=device, dtype=dt)
+    opv = op.transpose(-1, -2).contiguous().transpose(-1, -2)
+    stv = torch.stack([st, st], -1)[..., 0]
+    assert not opv.is_contiguous()
+    out = sim.apply_operator(op, qubits, st)
+    for a, b in ((opv, st), (op, stv), (opv, stv)):
+        ref = sim.apply_operator(a, qubits, b)
+        assert out.shape == ref.shape and out.dtype == ref.dtype and torch.equal(out, ref)
+    if dt.is_complex:
+        assert torch.equal(sim.apply_operator(op.conj(), qubits, st),
+                           sim.apply_operator(op.conj().resolve_conj(), qubits, st))
+    # phases: the state's own shape, one row, and a row behind a broadcast dim
+    for shape in {st.shape, (2 ** n,), (1, 2 ** n)}:
+        ang = torch.randn(shape, generator=g, device=device)
+        angv = torch.stack([ang, ang], -1)[..., 0]
+        got, ref = sim.apply_phase(ang, st), sim.apply_phase(angv, stv)
+        assert got.shape == ref.shape and got.dtype == ref.dtype
+        assert torch.allclose(got, ref, rtol=1e-6, atol=1e-7, equal_nan=True)
+
+
+def test_qubits_out_of_range_are_refused(device):
+    st = torch.randn(2 ** 4, dtype=torch.complex64, device=device)
+    op = torch.eye(2, dtype=torch.complex64, device=device)
+    for bad in ([4], [-1], [torch.tensor(2)], ["a"]):
+        with pytest.raises(ValueError):
+            sim.apply_operator(op, bad, st)
+    with pytest.raises(TypeError):
+        sim.apply_operator(op, [[1]], st)
