@@ -491,6 +491,10 @@ int ua_fused_pass_source(int dtype, int num_qubits, const ua_fused_pass* pass,
  * over groups is split across many workgroups; the float64 partial sums go to
  * `workspace` (ua_operator_gradient_workspace_bytes, 8-byte aligned; 0 bytes,
  * and NULL allowed, when one workgroup per result block suffices).
+ *
+ * ua_operator_backward -- that and the gradient w.r.t. the state for operators on
+ * 1 or 2 qubits, with one read of grad_out: grad_state (batch, 2^n), aliasing no
+ * input; state rows are contiguous (stride 2^n).  Same workspace.
  */
 #define UA_MAX_GRAD_QUBITS 16
 int64_t ua_operator_gradient_workspace_bytes(int num_qubits, int op_num_qubits, int64_t batch,
@@ -498,6 +502,10 @@ int64_t ua_operator_gradient_workspace_bytes(int num_qubits, int op_num_qubits, 
 int ua_operator_gradient(void* grad_op, const void* grad_out, const void* state, int dtype,
                          int num_qubits, int op_num_qubits, const int* qubits,
                          int64_t batch, int64_t op_count, int64_t state_batch_stride,
+                         void* workspace, ua_stream_t stream);
+int ua_operator_backward(void* grad_op, void* grad_state, const void* grad_out,
+                         const void* state, const void* op, int dtype, int num_qubits,
+                         int op_num_qubits, const int* qubits, int64_t batch, int64_t op_count,
                          void* workspace, ua_stream_t stream);
 
 /*

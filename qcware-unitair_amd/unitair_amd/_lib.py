@@ -69,6 +69,8 @@ SIGNATURES = {
     "ua_operator_gradient_workspace_bytes": (_i64, [_i32, _i32, _i64, _i64]),
     "ua_operator_gradient": (_i32, [_p, _p, _p, _i32, _i32, _i32, _pi32, _i64, _i64, _i64, _p,
                                     _p]),
+    "ua_operator_backward": (_i32, [_p, _p, _p, _p, _p, _i32, _i32, _i32, _pi32, _i64, _i64, _p,
+                                    _p]),
     "ua_pauli_gradients_workspace": (_i64, [_i32, _i64]),
     "ua_expect_sum_z": (_i32, [_p, _p, _i32, _i32, _i64, _p, _p]),
     "ua_apply_sum_z": (_i32, [_p, _p, _i32, _i32, _i64, _p]),

@@ -152,6 +152,7 @@ class _ApplyDense(torch.autograd.Function):
     Backward (derivation: out = U x on each group of amplitudes):
       grad_state = U^H grad_out          (ua_apply_operator, same kernel)
       grad_op    = sum grad_out x^H      (ua_operator_gradient)
+    or both in one pass (ua_operator_backward: 1- and 2-qubit operators).
     """
 
     @staticmethod
@@ -166,6 +167,12 @@ class _ApplyDense(torch.autograd.Function):
         qubits, n, k, out_batch, expand_state, op_bstride = ctx.meta
         g = grad_out.contiguous()
         grad_op = grad_state = None
+        if all(ctx.needs_input_grad[:2]) and k in (1, 2) and not expand_state and g.numel():
+            g = prepare(g)
+            grad_state = torch.empty_like(g)
+            grad_op = _operator_gradient(g, state, op, qubits, n, k, out_batch, False, op_bstride,
+                                         grad_state)
+            return grad_op, grad_state.reshape(state.shape), None, None, None, None, None, None
         if ctx.needs_input_grad[1]:
             op_h = op.conj().transpose(-1, -2).contiguous()
             full = _launch_operator(op_h, qubits, g, n, k, out_batch, False, op_bstride)
@@ -177,7 +184,10 @@ class _ApplyDense(torch.autograd.Function):
         return grad_op, grad_state, None, None, None, None, None, None
 
 
-def _operator_gradient(g, state, op, qubits, n, k, out_batch, expand_state, op_bstride):
+def _operator_gradient(g, state, op, qubits, n, k, out_batch, expand_state, op_bstride,
+                       grad_state=None):
+    """Gradient of the operator; with grad_state (a tensor like g) the state's
+    gradient goes there in the same pass."""
     lib = _lib.load()
     batch = math.prod(out_batch)
     N = 2 ** n
@@ -192,6 +202,14 @@ def _operator_gradient(g, state, op, qubits, n, k, out_batch, expand_state, op_b
     # a negative size flags bad arguments, which the entry point then reports
     nbytes = lib.ua_operator_gradient_workspace_bytes(n, k, batch, op_count)
     work = torch.empty(nbytes, dtype=torch.uint8, device=state.device) if nbytes > 0 else None
+    if grad_state is not None:
+        with on_device(state.device):
+            rc = lib.ua_operator_backward(
+                _lib.ptr(grad), _lib.ptr(grad_state), _lib.ptr(g), _lib.ptr(state), _lib.ptr(op),
+                _lib.DTYPE_CODES[state.dtype], n, k, _lib.int_array(qubits), batch, op_count,
+                _lib.ptr(work) if work is not None else None, _lib.stream_handle(state.device))
+        _lib.check(rc, "operator backward")
+        return grad
     with on_device(state.device):
         rc = lib.ua_operator_gradient(
             _lib.ptr(grad), _lib.ptr(g), _lib.ptr(s_flat.contiguous() if expand_state else s_flat),

@@ -265,3 +265,33 @@ def test_vqe_style_loss_through_drop_in_calls(device):
     loss(sim.apply_operator, ua.diag_expectation_value, tg, psi.to(device),
          h.to(device)).backward()
     assert torch.allclose(tg.grad.cpu(), tr.grad, atol=1e-11)
+
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128, torch.float32, torch.float64])
+@pytest.mark.parametrize("n,k,batch", [(1, 1, 3), (2, 2, 1), (3, 2, 5), (9, 1, 4), (13, 2, 3),
+                                       (16, 1, 2), (17, 2, 1)])
+@pytest.mark.parametrize("per_entry", [False, True])
+def test_operator_and_state_gradients_in_one_pass(device, dt, n, k, batch, per_entry):
+    """1- and 2-qubit operators: a backward that forms both gradients in one pass
+    gives the operator's bit for bit as when it is asked for alone, and the
+    state's as the adjoint operator applied to grad_out does (sums of 2^k products
+    in another order: at most 2 * 2^k roundings of the largest term)."""
+    g = torch.Generator(device=device).manual_seed(100 * n + 10 * k + batch)
+    qubits = torch.randperm(n, generator=torch.Generator().manual_seed(n))[:k].tolist()
+    op = torch.randn(((batch,) if per_entry else ()) + (2 ** k, 2 ** k), generator=g,
+                     device=device, dtype=dt)
+    st = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=dt)
+    go = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=dt)
+
+    def grads(a, b):
+        a, b = op.clone().requires_grad_(a), st.clone().requires_grad_(b)
+        need = [t for t in (a, b) if t.requires_grad]
+        return torch.autograd.grad(sim.apply_operator(a, qubits, b), need, go)
+    both_op, both_st = grads(True, True)
+    assert torch.equal(both_op, grads(True, False)[0])
+    alone = grads(False, True)[0]
+    assert both_st.shape == alone.shape == st.shape
+    eps = 2.0 ** -24 if dt in (torch.complex64, torch.float32) else 2.0 ** -53
+    largest = float(op.abs().max()) * float(go.abs().max())
+    assert float((both_st - alone).abs().max()) <= 4 * 2 ** k * eps * largest * 2 ** k
