@@ -220,8 +220,10 @@ def _program(items, n, dtype, device, compiled=False, key=None):
     # 12-bit tiles also for compiled passes: measured faster here than the
     # 13-bit default of compiled programs (34.5 vs 38.4 ms per step at 16
     # qubits x 1024 states)
+    # one_stream: a step's programs are built and run in one call, and autograd
+    # runs its backward on the stream of its forward
     return FusedProgram.from_items(items, n, dtype, device, tile_bits=12, compiled=compiled,
-                                   template=template)
+                                   template=template, one_stream=True)
 
 
 def _check_inputs(params, observable, n, dtype, device):
@@ -242,7 +244,7 @@ def _check_inputs(params, observable, n, dtype, device):
 
 class _Programs:
     """Every fused program of one parameter set, built before any of them
-    runs (building uploads op records, which waits for the stream)."""
+    runs (building uploads op records and forms the per-state products)."""
 
     def __init__(self, spec, p, dtype, dev, backward: bool):
         n = spec.n

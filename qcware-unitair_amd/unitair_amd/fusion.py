@@ -602,6 +602,48 @@ class PlanTemplate:
         return _product(PlanTemplate.evaluate(recipe[1], items),
                         PlanTemplate.evaluate(recipe[2], items))
 
+    @staticmethod
+    def evaluate_all(recipes, items):
+        """evaluate() of every recipe.  Per-state products of two input gates of
+        which one is diagonal, the usual kind, are formed together: scaled
+        columns or rows of one stacked tensor instead of a launch or three for
+        each (entries that are real or imaginary, as a rotation's are, come out
+        the same to the bit)."""
+        batches = {}     # (dense gate first, shape, dtype) -> [(position, dense, diagonal)]
+        alone = {}       # (shape, dtype) -> [(position, diagonal)] as 2x2 matrices
+        out = [None] * len(recipes)
+        for pos, r in enumerate(recipes):
+            if r[0] == "product":
+                kinds = [x[0] if x[0] == "item" else
+                         "diag" if x[0] == "as_dense1" and x[1][0] == "item" else None
+                         for x in r[1:]]
+                if sorted(map(str, kinds)) == ["diag", "item"]:
+                    first = kinds[0] == "item"          # the dense gate is the later one
+                    dense = items[r[1 if first else 2][1]]
+                    diag = items[r[2 if first else 1][1][1]]
+                    if dense.per_state and diag.per_state and diag.kind == "diag1" and \
+                            dense.kind == "dense1":
+                        key = (first, dense.data.shape, dense.data.dtype)
+                        batches.setdefault(key, []).append((pos, dense, diag))
+                        continue
+            elif r[0] == "as_dense1" and r[1][0] == "item":
+                diag = items[r[1][1]]
+                if diag.per_state and diag.kind == "diag1":
+                    alone.setdefault((diag.data.shape, diag.data.dtype), []).append((pos, diag))
+                    continue
+            out[pos] = PlanTemplate.evaluate(r, items)
+        for group in alone.values():
+            m = torch.diag_embed(torch.stack([g.data for _, g in group]))
+            for i, (pos, g) in enumerate(group):
+                out[pos] = _Item("dense1", g.bits, m[i], True)
+        for (first, _, _), group in batches.items():
+            m = torch.stack([g.data for _, g, _ in group])             # (R, B, 2, 2)
+            d = torch.stack([g.data for _, _, g in group])             # (R, B, 2)
+            prod = m * d.unsqueeze(-2 if first else -1)
+            for i, (pos, g, _) in enumerate(group):
+                out[pos] = _Item("dense1", g.bits, prod[i], True)
+        return out
+
 
 def _structure_key(code: int, n: int, fp, host_ops: int) -> tuple:
     """What a compiled pass depends on: dtype, n, the pass record and the kind
@@ -689,18 +731,21 @@ class FusedProgram:
                    device="cuda", tile_bits: Optional[int] = None,
                    reorder: bool = True, compiled: bool = False,
                    phase_angles: bool = False,
-                   template: Optional[PlanTemplate] = None) -> "FusedProgram":
-        """template: a PlanTemplate of an item list with the same kinds, bits
+                   template: Optional[PlanTemplate] = None,
+                   one_stream: bool = False) -> "FusedProgram":
+        """one_stream: the program is only run on the stream that is current
+        now, so that its upload need not be waited for.
+        template: a PlanTemplate of an item list with the same kinds, bits
         and per-state flags (its n, tile_bits and reorder apply); the plan is
         then taken from it instead of planned again."""
         prog = cls.__new__(cls)
         prog._build(list(items), n, dtype, device, tile_bits, reorder, compiled, phase_angles,
-                    template)
+                    template, one_stream)
         prog.num_gates = len(items)
         return prog
 
     def _build(self, items, n, dtype, device, tile_bits, reorder=True, compiled=False,
-               phase_angles=False, template=None):
+               phase_angles=False, template=None, one_stream=False):
         if tile_bits is None:
             # compiled passes take larger tiles (fewer passes); the interpreter 12
             tile_bits = COMPILED_TILE_BITS.get(dtype, TILE_BITS) if compiled else TILE_BITS
@@ -727,7 +772,8 @@ class FusedProgram:
             template.check(items)
         # fresh op records per program (data pointers differ between programs)
         op_structs = [FusedOp.from_buffer_copy(o) for o in template.op_structs]
-        pending = [(idx, PlanTemplate.evaluate(r, items)) for idx, r in template.pending]
+        pending = list(zip([idx for idx, _ in template.pending],
+                           PlanTemplate.evaluate_all([r for _, r in template.pending], items)))
         self._keep = []
         self.steps = []
         for st in template.steps:
@@ -770,7 +816,14 @@ class FusedProgram:
         arr = (FusedOp * max(1, len(op_structs)))(*op_structs)
         self._host_ops = arr
         raw = torch.frombuffer(bytearray(bytes(arr)), dtype=torch.uint8)
-        self._ops_dev = raw.to(self.device)
+        if one_stream and not torch.cuda.is_current_stream_capturing():
+            # from pinned memory (torch keeps it until the copy is done): a copy of
+            # pageable memory waits for everything queued on the stream
+            self._ops_dev = raw.pin_memory().to(self.device, non_blocking=True)
+        else:
+            # complete on return: any stream may run the program, or capture it
+            # (building while capturing is refused here)
+            self._ops_dev = raw.to(self.device)
         base_ptr = self._ops_dev.data_ptr()
         self._calls = []
         for st in self.steps:

@@ -222,3 +222,38 @@ def test_compiled_every_gate_of_a_cube(device, n, batch):
     ref = np.stack([oc.run_closed_form(gates, p) for p in psi])
     out = prog.run(torch.from_numpy(psi).to(device, torch.complex64)).cpu().numpy()
     assert rel_err(out, ref) < 1e-5
+
+
+def test_plan_recipes_together_match_one_by_one(device):
+    """PlanTemplate.evaluate_all against evaluate: per-state rotations (real or
+    imaginary entries: the same bits), general per-state gates (rounding) and
+    single diagonals, shared and per-state."""
+    from unitair_amd.fusion import PlanTemplate, _Item
+    g = torch.Generator(device=device).manual_seed(8)
+    B = 5
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device=device, dtype=torch.complex64)
+    t = torch.randn(B, generator=g, device=device)
+    c, s = torch.cos(t), torch.sin(t)
+    rot = torch.stack([torch.stack([c, -s], -1), torch.stack([s, c], -1)], -2).to(torch.complex64)
+    items = [_Item("diag1", (0,), torch.polar(torch.ones(B, 2, device=device),
+                                              rnd(B, 2).real).contiguous(), True),
+             _Item("dense1", (0,), rot.contiguous(), True),
+             _Item("dense1", (1,), rnd(B, 2, 2), True), _Item("diag1", (1,), rnd(B, 2), True),
+             _Item("diag1", (2,), np.array([1, 1j]), False), _Item("dense1", (2,), np.eye(2), False)]
+    d = lambda i: ("as_dense1", ("item", i))
+    recipes = [("product", ("item", 1), d(0)), ("product", d(0), ("item", 1)), d(0), d(3),
+               ("product", ("item", 2), d(3)), ("product", d(3), ("item", 2)), ("item", 2), d(4),
+               ("product", ("item", 5), d(4)), ("product", d(3), ("product", d(3), ("item", 2)))]
+    got = PlanTemplate.evaluate_all(recipes, items)
+    for i, (r, a) in enumerate(zip(recipes, got)):
+        b = PlanTemplate.evaluate(r, items)
+        assert (a.kind, a.bits, a.per_state) == (b.kind, b.bits, b.per_state)
+        x, y = torch.as_tensor(a.data), torch.as_tensor(b.data)
+        assert x.shape == y.shape and x.dtype == y.dtype
+        assert not isinstance(a.data, torch.Tensor) or a.data.is_contiguous()
+        if i < 4:
+            assert torch.equal(x, y)
+        else:
+            assert torch.allclose(x, y, rtol=1e-6, atol=1e-6)
