@@ -471,6 +471,11 @@ int ua_load_compiled_pass(void* handle);
  * structure. */
 int ua_run_compiled_pass(void* handle, void* state, int64_t batch, const ua_fused_op* ops,
                          ua_stream_t stream);
+/* The same with the first src_batch states read from src (contiguous, disjoint
+ * from all of state) and written to state: out of place for those states, in
+ * place for the others.  src_batch 0: ua_run_compiled_pass. */
+int ua_run_compiled_pass_from(void* handle, void* state, int64_t batch, const void* src,
+                              int64_t src_batch, const ua_fused_op* ops, ua_stream_t stream);
 /* The generated source of a pass's kernel (for inspection): *length gets its
  * size in bytes; up to capacity - 1 bytes and a terminating NUL go to buf. */
 int ua_fused_pass_source(int dtype, int num_qubits, const ua_fused_pass* pass,

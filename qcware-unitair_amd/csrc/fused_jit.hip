@@ -421,7 +421,7 @@ std::string generate(const PassShape& ps) {
   s << "extern \"C\" __global__ __launch_bounds__(" << threads
     << ") __attribute__((amdgpu_waves_per_eu("
     << waves << ")))\nvoid ua_compiled_pass(T* __restrict__ state, "
-    << "const OpRec* __restrict__ ops_arg) {\n";
+    << "const OpRec* __restrict__ ops_arg, const T* src, long long src_batch) {\n";
   s << "  const SC OpRec* ops = (const SC OpRec*)ops_arg;\n"
     << "  const int tid = threadIdx.x;\n"
     << "  const u64 tg = blockIdx.x;\n"
@@ -431,7 +431,11 @@ std::string generate(const PassShape& ps) {
   for (int i = 0; i < tbits; ++i)
     s << "  origin = ((origin >> " << local[i] << ") << " << local[i] + 1 << ") | (origin & "
       << hex64((uint64_t(1) << local[i]) - 1) << ");\n";
+  // states below src_batch are read from src and written to state: a copy of
+  // a checkpoint or of a state kept as one costs nothing beside the pass
   s << "  GL T* const st = (GL T*)state + b * " << hex64(uint64_t(1) << n) << ";\n"
+    << "  const GL T* const sr = (const GL T*)(b < src_batch ? src : state) + b * "
+    << hex64(uint64_t(1) << n) << ";\n"
     << "  const int t2 = 2 * tid;\n"
     << "  const u64 dep_t = u64(t2 & 15)";
   for (int i = 4; i < tbits - 3; ++i)
@@ -592,7 +596,7 @@ std::string generate(const PassShape& ps) {
       s << "    const int base = lds_pos(e0) * int(sizeof(T));\n";
     if (from_global) {
       for (int j = 0; j < 16; j += 2)
-        s << "    ld2(st + (gb | " << hex64(dep_j(j)) << "), q[" << j << "], q[" << j + 1
+        s << "    ld2(sr + (gb | " << hex64(dep_j(j)) << "), q[" << j << "], q[" << j + 1
           << "]);\n";
       if (head)
         for (int j = 0; j < 16; j += 2) {
@@ -675,7 +679,7 @@ std::string generate(const PassShape& ps) {
   } else {
     s << "  T c[16];\n";
     for (int k = 0; k < 8; ++k)
-      s << "  ld2(st + (origin | " << hex64(depk[k]) << " | dep_t), c[" << 2 * k << "], c["
+      s << "  ld2(sr + (origin | " << hex64(depk[k]) << " | dep_t), c[" << 2 * k << "], c["
         << 2 * k + 1 << "]);\n";
     if (head) diag_regs(0);
     if (uses_lds) {
@@ -879,6 +883,12 @@ extern "C" int ua_load_compiled_pass(void* handle) {
 
 extern "C" int ua_run_compiled_pass(void* handle, void* state, int64_t batch,
                                     const ua_fused_op* ops, ua_stream_t stream) {
+  return ua_run_compiled_pass_from(handle, state, batch, nullptr, 0, ops, stream);
+}
+
+extern "C" int ua_run_compiled_pass_from(void* handle, void* state, int64_t batch,
+                                         const void* src, int64_t src_batch,
+                                         const ua_fused_op* ops, ua_stream_t stream) {
   UA_CHECK_ARG(handle != nullptr, "NULL handle");
   auto* c = static_cast<ua::Compiled*>(handle);
   UA_CHECK_ARG(batch >= 0, "negative batch");
@@ -887,11 +897,23 @@ extern "C" int ua_run_compiled_pass(void* handle, void* state, int64_t batch,
   UA_CHECK_ARG(reinterpret_cast<uintptr_t>(state) % (2 * ua::elem_size(c->dtype)) == 0,
                "state must be aligned to two elements");
   const int64_t blocks = batch << (c->n - c->tile_bits);
+  UA_CHECK_ARG(src_batch >= 0 && src_batch <= batch, "src_batch must be 0..batch");
+  if (src_batch > 0) {
+    UA_CHECK_ARG(src != nullptr, "NULL pointer");
+    UA_CHECK_ARG(reinterpret_cast<uintptr_t>(src) % (2 * ua::elem_size(c->dtype)) == 0,
+                 "src must be aligned to two elements");
+    // a tile may be written before another one is read
+    const uintptr_t a = reinterpret_cast<uintptr_t>(src), d = reinterpret_cast<uintptr_t>(state);
+    const uintptr_t one = uintptr_t(ua::elem_size(c->dtype)) << c->n;
+    UA_CHECK_ARG(a + uintptr_t(src_batch) * one <= d || d + uintptr_t(batch) * one <= a,
+                 "src and state overlap");
+  }
   UA_CHECK_ARG(batch <= (int64_t(0x7fffffff) >> (c->n - c->tile_bits)), "too many tiles");
   hipFunction_t f = nullptr;
   const int rc = ua::function_of(c, &f);
   if (rc != UA_OK) return rc;
-  void* args[] = {&state, &ops};
+  long long from = src_batch;
+  void* args[] = {&state, &ops, &src, &from};
   const unsigned threads = 1u << (c->tile_bits - 4);
   const hipError_t e = hipModuleLaunchKernel(f, unsigned(blocks), 1, 1, threads, 1, 1, 0,
                                              static_cast<hipStream_t>(stream), args, nullptr);

@@ -874,16 +874,37 @@ class FusedProgram:
                 self._calls[i] = ("compiled", _COMPILED[keys[i]], self._calls[i][2])
         self.num_compiled = len(todo)
 
-    def run(self, state: torch.Tensor) -> torch.Tensor:
-        """Apply the program to a contiguous (batch, 2**n) state in place."""
+    def run(self, state: torch.Tensor, source: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """Apply the program to a contiguous (batch, 2**n) state in place.
+        source: a contiguous (m, 2**n) tensor apart from state that holds the
+        first m states' input (m <= batch); it is left as it is.  A compiled
+        first pass reads it in place of state, others copy it there first."""
         if state.device != self.device or state.dtype != self.dtype or \
                 state.shape[-1] != 2 ** self.n or not state.is_contiguous():
             raise ValueError("state must be a contiguous (batch, 2**n) tensor of the "
                              "program's dtype and device")
         batch = state.numel() // (2 ** self.n)
         stream = _lib.stream_handle(self.device)
+        m = 0
+        if source is not None:
+            m = source.numel() // (2 ** self.n)
+            if source.device != self.device or source.dtype != self.dtype or m > batch or \
+                    source.shape[-1] != 2 ** self.n or not source.is_contiguous():
+                raise ValueError("source must be a contiguous (m, 2**n) tensor of the "
+                                 "program's dtype and device, m <= batch")
+            d = source.data_ptr() - state.data_ptr()
+            if m and -m < d / (state.element_size() << self.n) < batch:
+                raise ValueError("source and state overlap")
+            if not (self._calls and self._calls[0][0] == "compiled"):
+                state.view(-1, 2 ** self.n)[:m].copy_(source.view(-1, 2 ** self.n))
+                m = 0
         for c in self._calls:
-            if c[0] == "compiled":
+            if c[0] == "compiled" and m:
+                rc = self.lib.ua_run_compiled_pass_from(c[1], _lib.ptr(state), batch,
+                                                        _lib.ptr(source), m,
+                                                        ctypes.c_void_p(c[2]), stream)
+                m = 0
+            elif c[0] == "compiled":
                 rc = self.lib.ua_run_compiled_pass(c[1], _lib.ptr(state), batch,
                                                    ctypes.c_void_p(c[2]), stream)
             elif c[0] == "fused":

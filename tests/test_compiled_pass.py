@@ -148,3 +148,22 @@ def test_compile_in_background_fills_the_table():
         assert _structure_key(_lib.UA_COMPLEX64, n, fp, ctypes.addressof(arr)) in fusion._COMPILED
     # a second request for the same structure compiles nothing
     assert fusion.compile_in_background(items, n, reorder=False).result(timeout=300) == 0
+
+
+def test_run_from_a_source_argument_checks():
+    """Refused before a device is touched: a count outside the batch, a NULL,
+    misaligned or overlapping source (the addresses are never read)."""
+    lib = _lib.load()
+    n = 14
+    passes, arr = _structs(random_mixed_circuit(n, 20, seed=2), n)
+    rc, h = _compile(lib, _lib.UA_COMPLEX64, n, *passes[0])
+    _lib.check(rc, "compile")
+    base, one = 1 << 20, 8 << n
+
+    def run(src, m, batch=3):
+        p = lambda v: ctypes.c_void_p(v or None)
+        return lib.ua_run_compiled_pass_from(p(h), p(base), batch, p(src), m, p(base), None)
+    for src, m in ((base + 8 * one, -1), (base + 8 * one, 4), (0, 1), (base + 8 * one + 8, 1),
+                   (base, 1), (base + 3 * one - 16, 1), (base - one + 16, 1)):
+        assert run(src, m) == _lib.UA_ERR_INVALID_ARGUMENT, (src, m)
+    assert run(base + 8 * one, 1, 0) == _lib.UA_OK

@@ -257,3 +257,27 @@ def test_plan_recipes_together_match_one_by_one(device):
             assert torch.equal(x, y)
         else:
             assert torch.allclose(x, y, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("compiled", [False, True])
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n,batch,m", [(8, 2, 1), (12, 3, 1), (13, 4, 4), (16, 3, 2), (16, 2, 0)])
+def test_run_from_a_source(device, dt, n, batch, m, compiled):
+    """The first m states read from another tensor, which stays as it is: the
+    same bits as a copy and a run in place (several pass structures each)."""
+    g = torch.Generator(device=device).manual_seed(n)
+    x = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=dt)
+    src = torch.randn(m, 2 ** n, generator=g, device=device, dtype=dt)
+    for seed in (3, 4):
+        circ = random_mixed_circuit(n, 50, seed=seed)
+        prog = FusedProgram(circ, dtype=dt, device=device, compiled=compiled)
+        a, b, kept = x.clone(), x.clone(), src.clone()
+        a[:m] = src
+        prog.run(a)
+        prog.run(b, kept)
+        assert torch.equal(a, b) and torch.equal(kept, src)
+    with pytest.raises(ValueError):
+        prog.run(x, torch.zeros(batch + 1, 2 ** n, dtype=dt, device=device))
+    if compiled and n >= 12 and m:
+        with pytest.raises(ValueError, match="overlap"):
+            prog.run(x, x[batch - m:])
