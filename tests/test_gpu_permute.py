@@ -184,3 +184,29 @@ def test_entry_points_reject_bad_arguments(device):
                                    0, 0, 1, 16, s) == 1
     assert lib.ua_apply_controlled_flip(_lib.ptr(out), _lib.ptr(x), c64, 4, 0b0101, 2, 1, 16,
                                         s) == 1
+
+
+def _gathered(perm, x, n):
+    i = torch.arange(2 ** n, device=x.device)
+    src = torch.zeros_like(i)
+    for q in range(n):
+        src |= ((i >> (n - 1 - q)) & 1) << (n - 1 - perm[q])
+    return x[..., src]
+
+
+@pytest.mark.parametrize("dt", DTYPES)
+@pytest.mark.parametrize("n,batch", [(10, 1), (10, 33), (11, 3), (14, 2), (18, 1), (20, 9)])
+def test_permute_tiles(device, dt, n, batch):
+    """The tiled kernel and the general one (a state that starts one element off
+    the alignment of its accesses; complex128 beyond the cache) against an
+    index gather: reversal, rolls, a swap of the ends, random orders."""
+    rng = np.random.default_rng(n)
+    flat = torch.from_numpy(rand((batch * 2 ** n + 1,), dt, rng)).to(device)
+    ident = list(range(n))
+    perms = [ident[::-1], ident[1:] + ident[:1], ident[5:] + ident[:5],
+             [n - 1] + ident[1:-1] + [0], ident[:n - 7] + ident[n - 7:][::-1]]
+    perms += [[int(p) for p in rng.permutation(n)] for _ in range(4)]
+    for perm in perms:
+        for off in (0, 1):
+            x = flat[off:off + batch * 2 ** n].view(batch, 2 ** n)
+            assert torch.equal(sim.permute_qubits(perm, x), _gathered(perm, x, n)), (perm, off)
