@@ -97,6 +97,92 @@ __global__ __launch_bounds__(kBlock) void dense_xch_kernel(
   }
 }
 
+// 2- and 3-qubit gates whose targets all lie in the low 6 + k bits, so that
+// the 64 groups of a wavefront are one contiguous block of amplitudes: the
+// block moves in whole lines and is exchanged in LDS, where each lane finds
+// its group.  (With a thread reading its own group, targets on low bits make
+// every access of a wavefront touch 64 different lines.)  The operator is read
+// with scalar loads.  The products are those of dense_fast_kernel, in the same
+// order.  Bound by memory: 24 qubits complex64 41 us for 2 targets, 45 for 3
+// (6.5 and 6.0 TB/s) wherever they lie, 42..65 and 46..79 before.
+struct LowParams {
+  int64_t total;        // wavefronts that own work
+  int64_t in_bstride, out_bstride, op_bstride;
+  int log2_wps;         // log2(wavefronts per state)
+  int tb[3];            // ascending target bit positions
+  int gpos[3];          // gate-index bit of canonical bit p
+};
+
+template <typename T, int K>
+__global__ __launch_bounds__(kBlock) void dense_low_kernel(T* out, const T* in,
+                                                           const T* __restrict__ op,
+                                                           LowParams p) {
+  using A = Num<T>;
+  constexpr int D = 1 << K, C = 64 * D, V = sizeof(T) == 16 ? 1 : 2, M = D / V;
+  // log2 of the elements that span the LDS banks: higher bits are XORed in
+  constexpr int NB = sizeof(T) == 16 ? 4 : sizeof(T) == 8 ? 5 : 6;
+  __shared__ T tiles[kBlock / 64][C];
+  const int lane = threadIdx.x & 63;
+  T* tile = tiles[threadIdx.x >> 6];
+  const int64_t w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)) +
+                    int64_t(blockIdx.x) * (kBlock / 64);
+  if (w >= p.total) return;            // whole wavefronts; no workgroup barrier below
+  const int64_t b = w >> p.log2_wps;
+  const int64_t first = (w & ((int64_t(1) << p.log2_wps) - 1)) * C;
+  const T* src = in + b * p.in_bstride + first;
+  T* dst = out + b * p.out_bstride + first;
+  const T* u = op + b * p.op_bstride;
+  auto pos = [](int e) { return e ^ ((e >> NB) & ((1 << NB) - 1)); };
+  auto fence = []() {                  // LDS accesses of a wavefront complete in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  struct alignas(V * sizeof(T)) Unit { T v[V]; };
+  Unit x[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+    x[m] = *reinterpret_cast<const Unit*>(src + (m * 64 + lane) * V);
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int h = 0; h < V; ++h) tile[pos((m * 64 + lane) * V + h)] = x[m].v[h];
+  fence();
+  int base = lane;
+#pragma unroll
+  for (int q = 0; q < K; ++q)
+    base = ((base >> p.tb[q]) << (p.tb[q] + 1)) | (base & ((1 << p.tb[q]) - 1));
+  int off[D], orig[D];                 // by canonical gate index
+#pragma unroll
+  for (int j = 0; j < D; ++j) {
+    off[j] = orig[j] = 0;
+#pragma unroll
+    for (int q = 0; q < K; ++q)
+      if ((j >> q) & 1) {
+        off[j] |= 1 << p.tb[q];
+        orig[j] |= 1 << p.gpos[q];
+      }
+  }
+  const int pb = pos(base);            // pos is linear: pos(base | off) = pb ^ pos(off)
+  T a[D];
+#pragma unroll
+  for (int j = 0; j < D; ++j) a[j] = tile[pb ^ pos(off[j])];
+  fence();
+#pragma unroll
+  for (int r = 0; r < D; ++r) {
+    T acc = A::zero();
+#pragma unroll
+    for (int j = 0; j < D; ++j) acc = A::mac(acc, u[orig[r] * D + orig[j]], a[j]);
+    tile[pb ^ pos(off[r])] = acc;
+  }
+  fence();
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+#pragma unroll
+    for (int h = 0; h < V; ++h) x[m].v[h] = tile[pos((m * 64 + lane) * V + h)];
+    *reinterpret_cast<Unit*>(dst + (m * 64 + lane) * V) = x[m];
+  }
+}
+
 // Any k (including 0 and k > 5): one thread per output amplitude, reading
 // its group from memory.  Out of place only.
 constexpr int kMaxQubits = 62;
@@ -146,6 +232,17 @@ void launch_xch(void* out, const void* in, const void* op, const XchParams& p, i
     case 2: dense_xch_kernel<T, 2><<<grid_for(p.total, kBlock * 2), kBlock, 0, s>>>(o, i, m, p); break;
     default: dense_xch_kernel<T, 1><<<grid_for(p.total, kBlock), kBlock, 0, s>>>(o, i, m, p);
   }
+}
+
+template <typename T>
+void launch_low(int k, void* out, const void* in, const void* op, const LowParams& p,
+                hipStream_t s) {
+  T* o = static_cast<T*>(out);
+  const T* i = static_cast<const T*>(in);
+  const T* m = static_cast<const T*>(op);
+  const unsigned grid = grid_for(p.total, kBlock / 64);
+  if (k == 2) dense_low_kernel<T, 2><<<grid, kBlock, 0, s>>>(o, i, m, p);
+  else dense_low_kernel<T, 3><<<grid, kBlock, 0, s>>>(o, i, m, p);
 }
 
 bool aligned(const void* ptr, int64_t stride_elems, size_t esize, size_t align) {
@@ -242,6 +339,35 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
         case UA_COMPLEX128: launch_xch<double2>(out, state, op, x, unr, s); break;
       }
       return check_launch("dense_xch_kernel");
+    }
+    // Targets within a wavefront's block (dense_low_kernel).  Where the line
+    // lies (24 qubits, complex64, us by index bits of the targets; vector
+    // kernel -> this one):
+    //   3 targets      0 1 2  61 -> 45, 1 2 3  79 -> 45, 5 6 8  49 -> 44
+    //   2, one of 1..3 1 2    65 -> 42, 2 3    55 -> 41, 0 2    45 -> 42
+    //   2 others       0 5    41 -> 41, 4 6    43 -> 41 (20 qubits 3.6 -> 3.9)
+    // With one operator per state 12 qubits x 4096: 1 2  64 -> 41, 0 5  60 -> 41,
+    // 0 1 2  59 -> 45, but 5 6 8  43 -> 45.  A few wavefronts only (under 12
+    // qubits) wait longer for its three trips through LDS: 1.84 -> 1.95.
+    const int64_t low_waves = n >= k + 6 ? batch << (n - k - 6) : 0;
+    const bool line_bits = tb[0] <= 3 && (tb[0] > 0 || (k == 2 && tb[1] <= 3));
+    const bool low = k == 3 ? low_waves >= 64 && (op_bstride == 0 || tb[0] <= 3)
+                            : low_waves >= 16 && (line_bits || (op_bstride != 0 && tb[0] == 0));
+    if ((k == 2 || k == 3) && io_aligned && tb[k - 1] < k + 6 && low) {
+      LowParams l{};
+      l.log2_wps = n - k - 6;
+      l.total = batch << l.log2_wps;
+      l.in_bstride = state_bstride;
+      l.out_bstride = N;
+      l.op_bstride = op_bstride;
+      for (int m = 0; m < k; ++m) { l.tb[m] = tb[m]; l.gpos[m] = gp[m]; }
+      switch (dtype) {
+        case UA_FLOAT32: launch_low<float>(k, out, state, op, l, s); break;
+        case UA_FLOAT64: launch_low<double>(k, out, state, op, l, s); break;
+        case UA_COMPLEX64: launch_low<float2>(k, out, state, op, l, s); break;
+        case UA_COMPLEX128: launch_low<double2>(k, out, state, op, l, s); break;
+      }
+      return check_launch("dense_low_kernel");
     }
     int mode = SCALAR;
     if (io_aligned) mode = (tb[0] == 0) ? PAIR : VEC;

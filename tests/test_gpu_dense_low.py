@@ -1,0 +1,63 @@
+"""2- and 3-qubit gates whose targets lie within one wavefront's block of
+amplitudes (dense_low_kernel) against the oracle, and bit for bit against the
+general kernel, which takes the same products in the same order: it runs the
+same call on a state one element off the alignment."""
+import numpy as np
+import pytest
+import torch
+
+from unitair_amd import _lib
+from unitair_amd import simulation as sim
+from oracle import unitair_np as U
+
+pytestmark = pytest.mark.gpu
+
+# an output sums 2 * 2^k <= 16 products, each rounded once: 16 half-ulps of the
+# sum of their magnitudes, itself a few times the largest output
+TOL = {torch.float32: 4e-6, torch.complex64: 4e-6, torch.float64: 8e-15, torch.complex128: 8e-15}
+NP = {torch.complex64: np.complex64, torch.complex128: np.complex128,
+      torch.float32: np.float32, torch.float64: np.float64}
+# target index bits; per k: lowest, lines split, the block's last bit, beyond it
+BITS = {2: [(0, 1), (1, 2), (3, 0), (7, 2), (0, 7), (8, 1), (6, 4)],
+        3: [(0, 1, 2), (3, 1, 2), (8, 0, 7), (5, 8, 6), (4, 2, 0), (9, 1, 0)]}
+
+
+def _rand(shape, rng, dt):
+    x = rng.standard_normal(shape)
+    if dt.is_complex:
+        x = x + 1j * rng.standard_normal(shape)
+    return torch.from_numpy(np.asarray(x).astype(NP[dt]))
+
+
+@pytest.mark.parametrize("per_state", [False, True])
+@pytest.mark.parametrize("dt", list(TOL))
+@pytest.mark.parametrize("k,n,batch", [(2, 8, 33), (2, 10, 5), (2, 13, 1), (2, 12, 3),
+                                       (3, 9, 70), (3, 9, 63), (3, 11, 17), (3, 15, 1)])
+def test_low_targets(device, dt, k, n, batch, per_state):
+    rng = np.random.default_rng(100 * n + batch)
+    size = batch * 2 ** n
+    for bits in BITS[k]:
+        if max(bits) >= n:
+            continue
+        qubits = [n - 1 - b for b in bits]
+        ops = _rand(((batch,) if per_state else ()) + (2 ** k, 2 ** k), rng, dt)
+        st = _rand((batch, 2 ** n), rng, dt)
+        wide = {True: np.complex128, False: np.float64}[dt.is_complex]
+        ref = U.apply_operator(ops.numpy().astype(wide), qubits, st.numpy().astype(wide))
+        opd, x = ops.to(device), st.to(device)
+        out = sim.apply_operator(opd, qubits, x)
+        err = np.max(np.abs(out.cpu().numpy() - ref)) / np.max(np.abs(ref))
+        assert err < TOL[dt], (bits, err)
+        buf = torch.empty(2 * size + 4, dtype=dt, device=device)
+        off, res = buf[1:1 + size].view(batch, 2 ** n), buf[size + 1:2 * size + 1].view(batch, -1)
+        off.copy_(x)
+
+        def call(o, i):
+            _lib.check(_lib.load().ua_apply_operator(
+                _lib.ptr(o), _lib.ptr(i), _lib.ptr(opd), _lib.DTYPE_CODES[dt], n, k,
+                _lib.int_array(qubits), batch, 2 ** n, 4 ** k if per_state else 0,
+                _lib.stream_handle(device)), "apply_operator")
+        call(res, off)
+        assert torch.equal(res, out), bits
+        call(x, x)                                  # in place
+        assert torch.equal(x, out), bits
