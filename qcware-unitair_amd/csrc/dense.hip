@@ -309,12 +309,16 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
     for (int m = 0; m < k; ++m) { p.tb[m] = tb[m]; p.gpos[m] = gp[m]; }
     // Matrix cores for the fused-block sizes where they measured faster on
     // MI355X (28-qubit complex64 / 27-qubit complex128 states): every 5-qubit
-    // gate; complex128 4-qubit gates; complex64 4-qubit gates only when all
-    // targets lie in the low 6 bits (the vector kernel streams the others at
-    // HBM speed).
+    // gate; complex128 4-qubit gates; complex64 4-qubit gates when all targets
+    // lie in the low 6 bits (the vector kernel streams the others at HBM
+    // speed: 26 qubits 208..225 us, matrix cores 222..235) or the states stay
+    // in the caches, where the vector kernel waits for LDS and the matrix: 16
+    // qubits 8.6..12.9 -> 3.0 us, 22 qubits 16.6..20 -> 14.5..16.8 (23 qubits
+    // with several states in turn: 28..40 and 26..45, by the targets).
     const bool mfma_shape =
         (k == 5 && dtype != UA_FLOAT32 && dtype != UA_FLOAT64) ||
-        (k == 4 && dtype == UA_COMPLEX128) || (k == 4 && dtype == UA_COMPLEX64 && tb[k - 1] < 6);
+        (k == 4 && dtype == UA_COMPLEX128) || (k == 4 && dtype == UA_COMPLEX64 &&
+         (tb[k - 1] < 6 || batch <= ((int64_t(1) << 22) >> n)));
     if (g_use_mfma && mfma_shape && op_bstride == 0 && n - k >= 6)
       return apply_dense_mfma(out, state, op, dtype, n, k, tb, gp, batch, state_bstride, s);
 

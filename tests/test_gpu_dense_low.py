@@ -61,3 +61,30 @@ def test_low_targets(device, dt, k, n, batch, per_state):
         assert torch.equal(res, out), bits
         call(x, x)                                  # in place
         assert torch.equal(x, out), bits
+
+
+@pytest.mark.parametrize("n,batch", [(9, 2), (10, 1), (10, 4096), (10, 4097), (13, 7), (17, 3)])
+def test_4_qubit_gates_on_either_side_of_the_matrix_core_rule(device, n, batch):
+    """complex64 4-qubit gates: vector kernel under 10 qubits and beyond the
+    caches, matrix cores between, any targets and alignment, also in place."""
+    rng = np.random.default_rng(n)
+    g = torch.Generator(device=device).manual_seed(n)
+    pick = sorted({0, batch // 2, batch - 1})
+    for bits in [(0, 1, 5, 7), (8, 7, 6, n - 1), (n - 1, 3, 0, n - 3), (2, 4, 5, 7)]:
+        if len(set(bits)) < 4:
+            continue
+        qubits = [n - 1 - b for b in bits]
+        op = _rand((16, 16), rng, torch.complex64)
+        flat = torch.randn(batch * 2 ** n + 1, generator=g, device=device, dtype=torch.complex64)
+        for off in (0, 1):
+            x = flat[off:off + batch * 2 ** n].view(batch, 2 ** n)
+            ref = U.apply_operator(op.numpy().astype(np.complex128), qubits,
+                                   x[pick].cpu().numpy().astype(np.complex128))
+            out = sim.apply_operator(op.to(device), qubits, x)
+            err = np.max(np.abs(out[pick].cpu().numpy() - ref)) / np.max(np.abs(ref))
+            assert err < 8e-6, (bits, off, err)     # 32 products: as above, twice the terms
+            y, opd = x.clone(), op.to(device)
+            _lib.check(_lib.load().ua_apply_operator(
+                _lib.ptr(y), _lib.ptr(y), _lib.ptr(opd), _lib.UA_COMPLEX64, n, 4,
+                _lib.int_array(qubits), batch, 2 ** n, 0, _lib.stream_handle(device)), "in place")
+            assert torch.equal(y, out)
