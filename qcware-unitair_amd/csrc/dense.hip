@@ -97,10 +97,10 @@ __global__ __launch_bounds__(kBlock) void dense_xch_kernel(
   }
 }
 
-// 2- and 3-qubit gates whose targets all lie in the low 6 + k bits, so that
-// the 64 groups of a wavefront are one contiguous block of amplitudes: the
-// block moves in whole lines and is exchanged in LDS, where each lane finds
-// its group.  (With a thread reading its own group, targets on low bits make
+// 2- and 3-qubit gates with targets on low index bits.  A wavefront's 64 groups
+// are taken as one block of 2^(6 + k) amplitudes, contiguous but for the
+// targets beyond it, which are its highest bits: the block moves in whole
+// lines and is exchanged in LDS, where each lane finds its group.  (With a thread reading its own group, targets on low bits make
 // every access of a wavefront touch 64 different lines.)  The operator is read
 // with scalar loads.  The products are those of dense_fast_kernel, in the same
 // order.  Bound by memory: 24 qubits complex64 41 us for 2 targets, 45 for 3
@@ -109,7 +109,10 @@ struct LowParams {
   int64_t total;        // wavefronts that own work
   int64_t in_bstride, out_bstride, op_bstride;
   int log2_wps;         // log2(wavefronts per state)
-  int tb[3];            // ascending target bit positions
+  int log2_run;         // log2(contiguous amplitudes): 6 + k - targets beyond
+  int beyond;           // targets at log2_run and above ...
+  int hb[2];            // ... and their state bits, ascending
+  int tb[3];            // ascending target positions in the block
   int gpos[3];          // gate-index bit of canonical bit p
 };
 
@@ -128,7 +131,8 @@ __global__ __launch_bounds__(kBlock) void dense_low_kernel(T* out, const T* in,
                     int64_t(blockIdx.x) * (kBlock / 64);
   if (w >= p.total) return;            // whole wavefronts; no workgroup barrier below
   const int64_t b = w >> p.log2_wps;
-  const int64_t first = (w & ((int64_t(1) << p.log2_wps) - 1)) * C;
+  const int64_t first = int64_t(insert_zero_bits(
+      uint64_t(w & ((int64_t(1) << p.log2_wps) - 1)) << p.log2_run, p.hb, p.beyond));
   const T* src = in + b * p.in_bstride + first;
   T* dst = out + b * p.out_bstride + first;
   const T* u = op + b * p.op_bstride;
@@ -137,11 +141,21 @@ __global__ __launch_bounds__(kBlock) void dense_low_kernel(T* out, const T* in,
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
   };
+  // state offset of access m's first element: 64 V <= 128 <= 2^log2_run
+  // elements lie in one run
+  auto at = [&](int m) {
+    const int e = m * 64 * V;
+    uint64_t o = e & ((1 << p.log2_run) - 1);
+#pragma unroll
+    for (int i = 0; i < K - 1; ++i)
+      if (i < p.beyond) o |= uint64_t((e >> (p.log2_run + i)) & 1) << p.hb[i];
+    return o;
+  };
   struct alignas(V * sizeof(T)) Unit { T v[V]; };
   Unit x[M];
 #pragma unroll
   for (int m = 0; m < M; ++m)
-    x[m] = *reinterpret_cast<const Unit*>(src + (m * 64 + lane) * V);
+    x[m] = *reinterpret_cast<const Unit*>(src + at(m) + lane * V);
 #pragma unroll
   for (int m = 0; m < M; ++m)
 #pragma unroll
@@ -179,7 +193,7 @@ __global__ __launch_bounds__(kBlock) void dense_low_kernel(T* out, const T* in,
   for (int m = 0; m < M; ++m) {
 #pragma unroll
     for (int h = 0; h < V; ++h) x[m].v[h] = tile[pos((m * 64 + lane) * V + h)];
-    *reinterpret_cast<Unit*>(dst + (m * 64 + lane) * V) = x[m];
+    *reinterpret_cast<Unit*>(dst + at(m) + lane * V) = x[m];
   }
 }
 
@@ -344,34 +358,57 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
       }
       return check_launch("dense_xch_kernel");
     }
-    // Targets within a wavefront's block (dense_low_kernel).  Where the line
-    // lies (24 qubits, complex64, us by index bits of the targets; vector
-    // kernel -> this one):
+    // Targets on low index bits (dense_low_kernel).  Where the line lies (24
+    // qubits, complex64, us by index bits of the targets; vector kernel -> this
+    // one):
     //   3 targets      0 1 2  61 -> 45, 1 2 3  79 -> 45, 5 6 8  49 -> 44
     //   2, one of 1..3 1 2    65 -> 42, 2 3    55 -> 41, 0 2    45 -> 42
     //   2 others       0 5    41 -> 41, 4 6    43 -> 41 (20 qubits 3.6 -> 3.9)
     // With one operator per state 12 qubits x 4096: 1 2  64 -> 41, 0 5  60 -> 41,
-    // 0 1 2  59 -> 45, but 5 6 8  43 -> 45.  A few wavefronts only (under 12
+    // 0 1 2  59 -> 45, but 5 6 8  43 -> 45.  With targets beyond the block two on
+    // bits 1..3 (h the highest bit): h 1 2  64 -> 46, 26 qubits 250 -> 191;
+    // complex128 any: 23 qubits h 1  61 -> 43, h 0 1  62 -> 50; one alone gains
+    // nothing in complex64 (22 qubits h 1  13.9 -> 14.5) and loses in float32
+    // (45 -> 50), but does with one operator per state (h 1  48 -> 42).  A few wavefronts only (under 12
     // qubits) wait longer for its three trips through LDS: 1.84 -> 1.95.
-    const int64_t low_waves = n >= k + 6 ? batch << (n - k - 6) : 0;
-    const bool line_bits = tb[0] <= 3 && (tb[0] > 0 || (k == 2 && tb[1] <= 3));
-    const bool low = k == 3 ? low_waves >= 64 && (op_bstride == 0 || tb[0] <= 3)
-                            : low_waves >= 16 && (line_bits || (op_bstride != 0 && tb[0] == 0));
-    if ((k == 2 || k == 3) && io_aligned && tb[k - 1] < k + 6 && low) {
+    if ((k == 2 || k == 3) && io_aligned && n >= k + 6) {
       LowParams l{};
-      l.log2_wps = n - k - 6;
-      l.total = batch << l.log2_wps;
-      l.in_bstride = state_bstride;
-      l.out_bstride = N;
-      l.op_bstride = op_bstride;
-      for (int m = 0; m < k; ++m) { l.tb[m] = tb[m]; l.gpos[m] = gp[m]; }
-      switch (dtype) {
-        case UA_FLOAT32: launch_low<float>(k, out, state, op, l, s); break;
-        case UA_FLOAT64: launch_low<double>(k, out, state, op, l, s); break;
-        case UA_COMPLEX64: launch_low<float2>(k, out, state, op, l, s); break;
-        case UA_COMPLEX128: launch_low<double2>(k, out, state, op, l, s); break;
+      int near = 0;                  // targets inside the contiguous run
+      while (near < k && tb[near] < 6 + near + 1) ++near;
+      int line_bits = 0, lowest = 4; // targets on bits 1..3, the first of them
+      for (int m = k - 1; m >= 0; --m)
+        if (tb[m] >= 1 && tb[m] <= 3) ++line_bits, lowest = tb[m];
+      const int64_t waves = batch << (n - k - 6);
+      bool low;
+      if (near < k)
+        low = near > 0 && (line_bits >= 2 || (es == 16 && lowest < (k == 2 ? 4 : 3)) ||
+                           (op_bstride != 0 && k == 2 && es >= 8 && (line_bits || tb[0] == 0)));
+      else if (k == 3)
+        low = op_bstride == 0 || tb[0] <= 3;
+      else
+        low = line_bits || (op_bstride != 0 && tb[0] == 0);
+      low = low && waves >= (k == 3 ? 64 : 16);
+      if (low) {
+        l.beyond = k - near;
+        l.log2_run = 6 + near;
+        l.log2_wps = n - k - 6;
+        l.total = batch << l.log2_wps;
+        l.in_bstride = state_bstride;
+        l.out_bstride = N;
+        l.op_bstride = op_bstride;
+        for (int m = 0; m < k; ++m) {
+          l.tb[m] = m < near ? tb[m] : 6 + m;
+          l.gpos[m] = gp[m];
+          if (m >= near) l.hb[m - near] = tb[m];
+        }
+        switch (dtype) {
+          case UA_FLOAT32: launch_low<float>(k, out, state, op, l, s); break;
+          case UA_FLOAT64: launch_low<double>(k, out, state, op, l, s); break;
+          case UA_COMPLEX64: launch_low<float2>(k, out, state, op, l, s); break;
+          case UA_COMPLEX128: launch_low<double2>(k, out, state, op, l, s); break;
+        }
+        return check_launch("dense_low_kernel");
       }
-      return check_launch("dense_low_kernel");
     }
     int mode = SCALAR;
     if (io_aligned) mode = (tb[0] == 0) ? PAIR : VEC;

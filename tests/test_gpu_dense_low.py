@@ -18,8 +18,9 @@ TOL = {torch.float32: 4e-6, torch.complex64: 4e-6, torch.float64: 8e-15, torch.c
 NP = {torch.complex64: np.complex64, torch.complex128: np.complex128,
       torch.float32: np.float32, torch.float64: np.float64}
 # target index bits; per k: lowest, lines split, the block's last bit, beyond it
-BITS = {2: [(0, 1), (1, 2), (3, 0), (7, 2), (0, 7), (8, 1), (6, 4)],
-        3: [(0, 1, 2), (3, 1, 2), (8, 0, 7), (5, 8, 6), (4, 2, 0), (9, 1, 0)]}
+BITS = {2: [(0, 1), (1, 2), (3, 0), (7, 2), (0, 7), (8, 1), (6, 4), (11, 2), (9, 3), (1, 12)],
+        3: [(0, 1, 2), (3, 1, 2), (8, 0, 7), (5, 8, 6), (4, 2, 0), (9, 1, 0),
+            (10, 2, 7), (10, 1, 9), (14, 12, 3), (0, 14, 2), (3, 6, 13)]}
 
 
 def _rand(shape, rng, dt):
