@@ -12,6 +12,9 @@
 // evaluated at the point right after that gate.  Same-kind rotations on
 // different qubits commute, so one (lambda, psi) point serves every qubit of a
 // layer: ua_pauli_gradients returns all n values of a layer in one call.
+#include <algorithm>
+
+#include "mfma_common.h"
 #include "ua_common.h"
 
 namespace ua {
@@ -742,7 +745,8 @@ extern "C" int ua_expect_sum_z(double* out, const void* psi, int dtype, int num_
 // wavefront shuffles and LDS.  With one part the sums go straight to grad_op;
 // otherwise to the float64 workspace, and op_grad_finish_kernel adds the
 // parts (one workgroup per result entry).  k = 1, 2 take the whole result in one block (each amplitude read
-// once); larger k tile it 4 x 4.
+// once); larger k tile it 4 x 4 (most operators on 4 and 5 qubits:
+// op_grad_mfma_kernel).
 //
 // GS (k = 1, 2): the thread holds whole groups of grad_out, so it also forms the
 // state's gradient U^H grad_out of them: one read of grad_out less, and no
@@ -906,6 +910,125 @@ __global__ __launch_bounds__(kBlock) void op_grad_partial_kernel(
   }
 }
 
+// The same for operators on 4 qubits (complex) and 5 (complex64), 16 A = 2^k rows:
+// the whole result in one workgroup, on the matrix cores.  Four groups are the depth of a
+// v_mfma_f64_16x16x4f64: lane l holds row l % 16 (+ 16 a) of group l / 16 of G
+// and of X, as loaded, and G^T conj(X) is four real products for each pair of
+// 16-row blocks.  Every amplitude is read once (the 4 x 4 blocks above read it
+// 2^k / 4 times and convert it each time); products are float64 and exact for
+// complex64, as there.  Bound by memory and the float64 products together: 22
+// qubits x 3 states complex64, 4 targets 105..331 -> 47..62 us by the targets, 5
+// targets 169..784 -> 78..92; 21 qubits complex128, 4 targets 97..291 -> 57..68; 10
+// qubits x 301 operators of their own 84 -> 7.1.  (complex128 on 5 qubits would
+// take too many registers for sums as short as the ones it has.)
+// A lane takes UNR neighbouring groups, one for each step: with no target on
+// the lowest index bits (RUN) they are neighbours in memory too.
+template <typename T, int A, bool RUN>
+__global__ __launch_bounds__(kBlock) void op_grad_mfma_kernel(
+    T* __restrict__ grad_op, double* __restrict__ part_out, const T* __restrict__ gout,
+    const T* __restrict__ in, OpGradParams p) {
+  constexpr int D = 16 * A, K = 3 + A, kWaves = kBlock / 64, UNR = 4;
+  // complex128: sums of their own for each step of a run and each of the two
+  // products.  One long chain had twice the rounding error of the many short
+  // ones of the kernel above (7e-16 against 3.4e-16); so it is no larger (18
+  // qubits x 3: 2.2e-16 against 2.6e-16).
+  constexpr int S = sizeof(T) == 16 ? 2 * UNR : 1;
+  using M = Mfma<double>;
+  __shared__ double2 red[D * D];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int64_t part = int64_t(blockIdx.x) % p.parts, o = int64_t(blockIdx.x) / p.parts;
+  uint64_t off[A];
+#pragma unroll
+  for (int a = 0; a < A; ++a) off[a] = gate_offset(16 * a + (lane & 15), p);
+  const int gbits = p.n - p.k;
+  const int64_t N = int64_t(1) << p.n;
+  const int64_t u_begin = part * p.units_per_part;
+  int64_t u_end = u_begin + p.units_per_part;
+  if (u_end > p.units) u_end = p.units;
+  M::acc_t re[S][A][A], im[S][A][A];
+#pragma unroll
+  for (int s = 0; s < S; ++s)
+#pragma unroll
+    for (int a = 0; a < A; ++a)
+#pragma unroll
+      for (int c = 0; c < A; ++c) re[s][a][c] = im[s][a][c] = M::acc_t{0.0, 0.0, 0.0, 0.0};
+  struct alignas(16) Run { T v[UNR]; };
+  for (int64_t u0 = u_begin + 4 * UNR * wave; u0 < u_end; u0 += 4 * UNR * kWaves) {  // wave-uniform
+    Run g[A], x[A];
+    const int64_t u = u0 + UNR * (lane >> 4);
+#pragma unroll
+    for (int q = 0; q < (RUN ? 1 : UNR); ++q) {
+      const bool ok = u + q < u_end;            // RUN: for all UNR of them
+      const int64_t v = ok ? u + q : u_begin;   // past the end: zeros count for nothing
+      const int64_t b = (p.op_count == 1) ? (v >> gbits) : o;
+      const uint64_t base =
+          insert_zero_bits(uint64_t(v) & ((uint64_t(1) << gbits) - 1), p.sorted, K);
+#pragma unroll
+      for (int a = 0; a < A; ++a) {
+        const T* gp = gout + b * N + base + off[a];
+        const T* xp = in + b * p.in_bstride + base + off[a];
+        if constexpr (RUN) {
+          g[a] = *reinterpret_cast<const Run*>(gp);
+          x[a] = *reinterpret_cast<const Run*>(xp);
+          if (!ok) g[a] = x[a] = Run{};
+        } else {
+          g[a].v[q] = ok ? *gp : T{};
+          x[a].v[q] = ok ? *xp : T{};
+        }
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < UNR; ++q)
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int c = 0; c < A; ++c) {            // g * conj(x)
+          const double2 gv = as_d2(g[a].v[q]), xv = as_d2(x[c].v[q]);
+          const int s0 = q % S, s1 = (q + UNR) % S;
+          re[s0][a][c] = M::mma(gv.x, xv.x, re[s0][a][c]);
+          im[s0][a][c] = M::mma(gv.y, xv.x, im[s0][a][c]);
+          re[s1][a][c] = M::mma(gv.y, xv.y, re[s1][a][c]);
+          im[s1][a][c] = M::mma(-gv.x, xv.y, im[s1][a][c]);
+        }
+  }
+#pragma unroll
+  for (int h = S / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int s = 0; s < h; ++s)
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int c = 0; c < A; ++c) {
+          re[s][a][c] += re[s + h][a][c];
+          im[s][a][c] += im[s + h][a][c];
+        }
+  for (int w = 0; w < kWaves; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int a = 0; a < A; ++a)
+#pragma unroll
+        for (int c = 0; c < A; ++c)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            double2& e = red[(16 * a + M::row(lane, i)) * D + 16 * c + (lane & 15)];
+            e.x = (w ? e.x : 0.0) + re[0][a][c][i];
+            e.y = (w ? e.y : 0.0) + im[0][a][c][i];
+          }
+    }
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < D * D; e += kBlock) {
+    if (p.parts == 1) {
+      grad_op[o * D * D + e] = from_d2<T>(red[e]);
+    } else {
+      double* dst = part_out + ((o * p.parts + part) * D * D + e) * 2;
+      dst[0] = red[e].x;
+      dst[1] = red[e].y;
+    }
+  }
+}
+
 // One workgroup per (operator, entry): the threads split the parts, then
 // reduce with wavefront shuffles and LDS.
 template <typename T>
@@ -945,7 +1068,7 @@ struct OpGradShape {
   int64_t nblk, parts, units, units_per_part;
 };
 
-OpGradShape op_grad_shape(int n, int k, int64_t batch, int64_t op_count) {
+OpGradShape op_grad_shape(int n, int k, int64_t batch, int64_t op_count, bool mfma) {
   OpGradShape sh{};
   const int64_t D = int64_t(1) << k;
   sh.rb = sh.cb = int(D < 4 ? D : 4);
@@ -955,8 +1078,20 @@ OpGradShape op_grad_shape(int n, int k, int64_t batch, int64_t op_count) {
   const int64_t want = (4096 + op_count * sh.nblk - 1) / (op_count * sh.nblk);
   const int64_t most = (sh.units + kBlock * 16 - 1) / (kBlock * 16);
   sh.parts = want < most ? want : most;
+  if (mfma) {
+    // one workgroup a part (op_grad_mfma_kernel): four per CU for 4 qubits, two
+    // for 5 (half as many: complex64 6 % slower, complex128 chains of twice the
+    // length), each with at least 128 groups (with 256: 14 qubits 14 -> 20 us)
+    const int64_t fill = ((k == 4 ? 1024 : 512) + op_count - 1) / op_count;
+    const int64_t full = (sh.units + 127) / 128;
+    sh.parts = fill < full ? fill : full;
+  }
   if (sh.parts < 1) sh.parts = 1;
   sh.units_per_part = (sh.units + sh.parts - 1) / sh.parts;
+  if (mfma) {                        // whole runs of neighbouring groups in a part
+    sh.units_per_part = (sh.units_per_part + 15) / 16 * 16;
+    sh.parts = (sh.units + sh.units_per_part - 1) / sh.units_per_part;
+  }
   return sh;
 }
 
@@ -975,6 +1110,16 @@ void launch_op_grad(int rb, unsigned grid, T* grad, double* part, const T* g, co
     op_grad_partial_kernel<T, 4, 4, 2, false><<<grid, kBlock, 0, s>>>(grad, part, g, x, gs, op, p);
 }
 
+template <typename T, int A>
+void launch_op_grad_mfma(unsigned grid, T* grad, double* part, const T* g, const T* x,
+                         const OpGradParams& p, hipStream_t s) {
+  // a lane's four neighbouring groups as one run
+  const bool run = p.sorted[0] >= 2 && reinterpret_cast<uintptr_t>(g) % 16 == 0 &&
+                   reinterpret_cast<uintptr_t>(x) % 16 == 0 && p.in_bstride % 2 == 0;
+  if (run) op_grad_mfma_kernel<T, A, true><<<grid, kBlock, 0, s>>>(grad, part, g, x, p);
+  else op_grad_mfma_kernel<T, A, false><<<grid, kBlock, 0, s>>>(grad, part, g, x, p);
+}
+
 }  // namespace
 }  // namespace ua
 
@@ -985,9 +1130,12 @@ extern "C" int64_t ua_operator_gradient_workspace_bytes(int num_qubits, int op_n
       !(op_count == 1 || op_count == batch))
     return -1;
   if (batch == 0) return 0;
-  const ua::OpGradShape sh = ua::op_grad_shape(n, k, batch, op_count);
-  if (sh.parts == 1) return 0;
-  return op_count * sh.parts * (int64_t(1) << (2 * k)) * 2 * int64_t(sizeof(double));
+  // for whichever type: complex ones take the matrix cores
+  int64_t parts = ua::op_grad_shape(n, k, batch, op_count, false).parts;
+  if (k == 4 || k == 5)
+    parts = std::max(parts, ua::op_grad_shape(n, k, batch, op_count, true).parts);
+  if (parts == 1) return 0;
+  return op_count * parts * (int64_t(1) << (2 * k)) * 2 * int64_t(sizeof(double));
 }
 
 namespace ua {
@@ -1018,7 +1166,9 @@ int operator_gradient(void* grad_op, void* grad_state, const void* grad_out, con
   }
   for (int b = 0, m = 0; b < n; ++b)
     if ((seen >> b) & 1) p.sorted[m++] = b;
-  const OpGradShape sh = op_grad_shape(n, k, batch, op_count);
+  const bool mfma = (k == 4 && (dtype == UA_COMPLEX64 || dtype == UA_COMPLEX128)) ||
+                    (k == 5 && dtype == UA_COMPLEX64);
+  const OpGradShape sh = op_grad_shape(n, k, batch, op_count, mfma);
   p.parts = sh.parts;
   p.units = sh.units;
   p.units_per_part = sh.units_per_part;
@@ -1030,7 +1180,18 @@ int operator_gradient(void* grad_op, void* grad_state, const void* grad_out, con
   hipStream_t s = static_cast<hipStream_t>(stream);
   double* part = static_cast<double*>(workspace);
   const unsigned grid = unsigned(blocks);
-  switch (dtype) {
+  if (mfma) {
+    const unsigned mgrid = unsigned(op_count * sh.parts);
+    if (dtype == UA_COMPLEX128)
+      launch_op_grad_mfma<double2, 1>(mgrid, (double2*)grad_op, part, (const double2*)grad_out,
+                                      (const double2*)state, p, s);
+    else if (k == 4)
+      launch_op_grad_mfma<float2, 1>(mgrid, (float2*)grad_op, part, (const float2*)grad_out,
+                                     (const float2*)state, p, s);
+    else
+      launch_op_grad_mfma<float2, 2>(mgrid, (float2*)grad_op, part, (const float2*)grad_out,
+                                     (const float2*)state, p, s);
+  } else switch (dtype) {
     case UA_FLOAT32:
       launch_op_grad(sh.rb, grid, (float*)grad_op, part, (const float*)grad_out, (const float*)state,
                      (float*)grad_state, (const float*)op, p, s);

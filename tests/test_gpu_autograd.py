@@ -295,3 +295,26 @@ def test_operator_and_state_gradients_in_one_pass(device, dt, n, k, batch, per_e
     eps = 2.0 ** -24 if dt in (torch.complex64, torch.float32) else 2.0 ** -53
     largest = float(op.abs().max()) * float(go.abs().max())
     assert float((both_st - alone).abs().max()) <= 4 * 2 ** k * eps * largest * 2 ** k
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n,k,ob,sb", [(4, 4, (), ()), (5, 4, (3,), (3,)), (7, 5, (), (5,)),
+                                       (13, 4, (), (1,)), (10, 4, (9,), (9,)), (15, 4, (), (3,)),
+                                       (16, 5, (), ()), (11, 5, (2,), (2,)), (9, 4, (5,), ())])
+def test_operator_gradient_of_4_and_5_qubit_operators(device, dt, n, k, ob, sb):
+    """The matrix-core reduction: fewer groups than one step takes, parts that do
+    not divide evenly, one operator and one per entry, one state for several."""
+    torch.manual_seed(10 * n + k)
+    real = {torch.complex64: torch.float32, torch.complex128: torch.float64}[dt]
+    for qubits in (list(range(n - k, n)), torch.randperm(n)[:k].tolist()):
+        op = torch.randn(*ob, 2 ** k, 2 ** k, dtype=dt)
+        st = torch.randn(*sb, 2 ** n, dtype=dt)
+        ref = _grads_cpu(lambda o, s: T.apply_operator(o, qubits, s),
+                         op.to(torch.complex128), st.to(torch.complex128))
+        got = _grads_gpu(lambda o, s: sim.apply_operator(o, qubits, s), device, op, st)
+        # the sums are float64; the incoming gradient depends on the rounded
+        # output (2^k products of it), which bounds complex64
+        eps = torch.finfo(real).eps
+        for r, g in zip(ref, got):
+            scale = float(r.abs().max())
+            assert float((r - g.to(torch.complex128)).abs().max()) <= 2 ** (k + 3) * eps * scale
