@@ -168,7 +168,8 @@ class _ApplyDense(torch.autograd.Function):
         g = grad_out.contiguous()
         grad_op = grad_state = None
         if all(ctx.needs_input_grad[:2]) and k in (1, 2) and not expand_state and g.numel():
-            g = prepare(g)
+            # (saved-tensor hooks may give back other strides than were saved)
+            g, op, state = (prepare(t).contiguous() for t in (g, op, state))
             grad_state = torch.empty_like(g)
             grad_op = _operator_gradient(g, state, op, qubits, n, k, out_batch, False, op_bstride,
                                          grad_state)
@@ -191,7 +192,7 @@ def _operator_gradient(g, state, op, qubits, n, k, out_batch, expand_state, op_b
     lib = _lib.load()
     batch = math.prod(out_batch)
     N = 2 ** n
-    grad = torch.empty_like(op)
+    grad = torch.empty_like(op, memory_format=torch.contiguous_format)
     if batch == 0:
         return grad.zero_()
     if k > _lib.UA_MAX_GRAD_QUBITS:

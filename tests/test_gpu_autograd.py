@@ -318,3 +318,21 @@ def test_operator_gradient_of_4_and_5_qubit_operators(device, dt, n, k, ob, sb):
         for r, g in zip(ref, got):
             scale = float(r.abs().max())
             assert float((r - g.to(torch.complex128)).abs().max()) <= 2 ** (k + 3) * eps * scale
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 4])
+def test_saved_tensors_that_come_back_with_other_strides(device, k):
+    """Hooks that unpack to transposed memory change no gradient."""
+    torch.manual_seed(k)
+    n, B = 7, 3
+    qubits = [6, 0, 3, 5][:k]
+    op = torch.randn(B, 2 ** k, 2 ** k, dtype=torch.complex128)
+    st = torch.randn(B, 2 ** n, dtype=torch.complex128)
+
+    def other(t):
+        return t.transpose(-1, -2).contiguous().transpose(-1, -2) if t.dim() > 1 else t
+    ref = _grads_gpu(lambda o, s: sim.apply_operator(o, qubits, s), device, op, st)
+    with torch.autograd.graph.saved_tensors_hooks(other, lambda t: t):
+        got = _grads_gpu(lambda o, s: sim.apply_operator(o, qubits, s), device, op, st)
+    for r, g in zip(ref, got):
+        assert torch.equal(r, g)
