@@ -40,8 +40,8 @@ constexpr int kMinTileBits = 12;  // tiles below 12 bits stay with the interpret
 int max_tile_bits(int dtype) { return dtype == UA_COMPLEX128 ? 13 : 14; }
 
 // Waves per SIMD the compiled complex64 kernels ask the register allocator
-// for (0: 4, the default; a complex64 tile takes 32 KiB of LDS, so at most
-// five workgroups of four waves fit a CU).  complex128 kernels ask for 2.
+// for (0: 4, and 5 for 12-bit tiles, whose 32 KiB fit a CU's LDS five times).
+// complex128 kernels ask for 2.
 std::atomic<int> g_compiled_waves{0};
 
 // Device code shared by every compiled pass.  UA_DOUBLE selects complex128.
@@ -417,7 +417,9 @@ std::string generate(const PassShape& ps) {
   const bool mfma = !dbl && tbits > 12;
   s << "#define UA_DOUBLE " << (dbl ? 1 : 0) << "\n#define UA_MFMA " << (mfma ? 1 : 0)
     << "\n#define UA_STREAM_PHASES " << (n >= (dbl ? 21 : 22) ? 1 : 0) << "\n" << kPrelude;
-  const int waves = dbl ? 2 : (g_compiled_waves > 0 ? int(g_compiled_waves) : 4);
+  // five 12-bit tiles fit a CU's LDS (16 qubits x 1024 states, a gradient step of
+  // 30 passes: 21.46 -> 21.27 ms)
+  const int waves = dbl ? 2 : g_compiled_waves > 0 ? int(g_compiled_waves) : tbits == 12 ? 5 : 4;
   s << "extern \"C\" __global__ __launch_bounds__(" << threads
     << ") __attribute__((amdgpu_waves_per_eu("
     << waves << ")))\nvoid ua_compiled_pass(T* __restrict__ state, "
