@@ -165,11 +165,11 @@ class _ApplyDense(torch.autograd.Function):
     def backward(ctx, grad_out):
         op, state = ctx.saved_tensors
         qubits, n, k, out_batch, expand_state, op_bstride = ctx.meta
-        g = grad_out.contiguous()
+        # a gradient may arrive lazily conjugated (a loss through out.conj()), and
+        # saved-tensor hooks may give back other strides than were saved
+        g, op, state = (prepare(t).contiguous() for t in (grad_out, op, state))
         grad_op = grad_state = None
         if all(ctx.needs_input_grad[:2]) and k in (1, 2) and not expand_state and g.numel():
-            # (saved-tensor hooks may give back other strides than were saved)
-            g, op, state = (prepare(t).contiguous() for t in (g, op, state))
             grad_state = torch.empty_like(g)
             grad_op = _operator_gradient(g, state, op, qubits, n, k, out_batch, False, op_bstride,
                                          grad_state)

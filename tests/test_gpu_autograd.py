@@ -336,3 +336,31 @@ def test_saved_tensors_that_come_back_with_other_strides(device, k):
         got = _grads_gpu(lambda o, s: sim.apply_operator(o, qubits, s), device, op, st)
     for r, g in zip(ref, got):
         assert torch.equal(r, g)
+
+
+@pytest.mark.parametrize("ob,sb,qubits", [((), (3,), (2,)), ((), (3,), (4, 0)), ((3,), (3,), (1, 3)),
+                                          ((), (), (3, 1, 2)), ((), (3,), (0, 4, 2, 1)),
+                                          ((4,), (), (0,)), ((4,), (), (3, 2)),
+                                          ((2,), (), (4, 1, 2))])
+@pytest.mark.parametrize("wrt", [(True, True), (True, False), (False, True)])
+def test_gradients_that_arrive_lazily_conjugated(device, ob, sb, qubits, wrt):
+    """A loss through out.conj() hands the backward a tensor with the conj bit
+    set: same gradients as the reference's, whichever inputs ask for one."""
+    torch.manual_seed(len(qubits))
+    n, k = 5, len(qubits)
+    op = torch.randn(*ob, 2 ** k, 2 ** k, dtype=torch.complex128)
+    st = torch.randn(*sb, 2 ** n, dtype=torch.complex128)
+    v = torch.randn(*(sb or ob), 2 ** n, dtype=torch.complex128)
+
+    def grads(fn, dev):
+        xs = [x.to(dev).requires_grad_(w) for x, w in zip((op.clone(), st.clone()), wrt)]
+        seen = []
+        out = fn(*xs)
+        out.register_hook(lambda g: seen.append(g.is_conj()))
+        loss = (out.conj() * v.to(dev)).imag.sum()
+        got = torch.autograd.grad(loss, [x for x in xs if x.requires_grad])
+        assert seen == [True]
+        return [g.resolve_conj().cpu() for g in got]
+    ref = grads(lambda o, s: T.apply_operator(o, qubits, s), "cpu")
+    for r, g in zip(ref, grads(lambda o, s: sim.apply_operator(o, qubits, s), device)):
+        assert torch.allclose(r, g, atol=1e-10)
