@@ -100,11 +100,13 @@ __global__ __launch_bounds__(kBlock) void dense_xch_kernel(
 // 2- and 3-qubit gates with targets on low index bits.  A wavefront's 64 groups
 // are taken as one block of 2^(6 + k) amplitudes, contiguous but for the
 // targets beyond it, which are its highest bits: the block moves in whole
-// lines and is exchanged in LDS, where each lane finds its group.  (With a thread reading its own group, targets on low bits make
-// every access of a wavefront touch 64 different lines.)  The operator is read
-// with scalar loads.  The products are those of dense_fast_kernel, in the same
-// order.  Bound by memory: 24 qubits complex64 41 us for 2 targets, 45 for 3
-// (6.5 and 6.0 TB/s) wherever they lie, 42..65 and 46..79 before.
+// lines and is exchanged in LDS, where each lane finds its group.  (With a
+// thread reading its own group, targets on low bits make every access of a
+// wavefront touch 64 different lines.)  The operator is read with scalar
+// loads.  The products are those of dense_fast_kernel, in the same order.
+// Bound by memory: 24 qubits complex64 41 us for 2 targets, 45 for 3 (6.5 and
+// 6.0 TB/s) wherever they lie, 42..65 and 46..79 before.  low_pays_2 and
+// low_pays_3 say where it is the faster one.
 struct LowParams {
   int64_t total;        // wavefronts that own work
   int64_t in_bstride, out_bstride, op_bstride;
@@ -264,6 +266,110 @@ bool aligned(const void* ptr, int64_t stride_elems, size_t esize, size_t align) 
          ((stride_elems * int64_t(esize)) % int64_t(align)) == 0;
 }
 
+// Where dense_low_kernel beats the vector kernel: by ratios of times measured for
+// 34 sets of targets from 2^10 to 2^28 amplitudes in each of the four types, with
+// one operator and one per state; ratios of 1 and above stay out.  What it saves
+// are the partial lines of targets on bits 1..3 ("lines"), so the wider the
+// element the more; what it adds are two trips through LDS and, with an operator
+// for each state, scalar loads that every wavefront waits for.  In between lies
+// the size: small states wait for the vector kernel's longer chain of accesses,
+// states beyond the Infinity Cache for their lines, those that it holds for
+// neither.  Measurements in us (vector kernel -> this one) are of complex64 states
+// of 24 qubits unless said otherwise, ratios are the range over the sizes.
+struct LowCase {
+  size_t es;       // bytes of an element
+  const int* tb;   // ascending targets, the first `near` of them inside the block
+  int near;
+  int64_t amps;    // all states together
+  bool per;        // an operator for each state
+  bool staged;     // the vector kernel would keep that in LDS (k = 3)
+  bool from(int e) const { return amps >= (int64_t(1) << e); }
+  bool up_to(int e) const { return amps < (int64_t(3) << e) / 2; }
+  bool beyond() const { return amps * int64_t(es) >= (int64_t(1) << 28); }
+};
+
+bool low_pays_2(const LowCase& c) {
+  const int* tb = c.tb;
+  const size_t es = c.es;
+  const bool near = c.near == 2;
+  int lines = 0, first = 4;
+  for (int m = 1; m >= 0; --m)
+    if (tb[m] >= 1 && tb[m] <= 3) ++lines, first = tb[m];
+  // float32: 1 2 0.79..0.95 (0.68 beyond the cache; per state up to 1.17 there); 1 5
+  // and 0 1 up to 1.21, 0.91 beyond
+  if (es == 4) {
+    if (c.per) return lines == 2 && c.from(18) && !c.beyond();
+    return lines == 2 || (lines && near && c.beyond());
+  }
+  if (tb[0] != 0) {
+    // 1 2 65 -> 42, 2 3 55 -> 41; bit 3 as the lowest 0.92 up to 2^18, then up to
+    // 1.15, 0.96 beyond (complex128 0.75..0.98 throughout).  Targets beyond the
+    // block: h 1 at 22 qubits 13.9 -> 14.0, with an operator per state 48 -> 46,
+    // complex128 at 23 qubits 61 -> 43
+    if (!near && !c.per && es == 8) return false;
+    return lines && (first < 3 || es == 16 || c.beyond() || (!c.per && c.up_to(18)));
+  }
+  // bit 0, which the vector kernel pairs: 0 1 and 0 2 0.94..0.98 from 2^19 (1.02
+  // below), 0 3 up to 1.12 within the cache; per state 10 qubits 0.80..0.93 from
+  // 2^19, 1.10 below.  complex128: 0 1 0.64..0.94, others 1.04 below 2^19
+  if (es == 16 && tb[1] == 1) return true;
+  if (!c.from(19)) return false;
+  if (c.per) return es == 8 || lines || c.up_to(21);
+  return near && tb[1] <= (es == 16 || c.beyond() ? 3 : 2);
+}
+
+// Where the vector kernel keeps each state's operator in LDS that beats the scalar
+// loads unless lines are saved (0 1 5 with 12 qubits x 64: 1.57); where it reads
+// the operator from memory (10 qubits x 8192: 0.36..0.9) nearly everything gains.
+bool low_pays_3(const LowCase& c) {
+  const int* tb = c.tb;
+  const bool near = c.near == 3, per = c.per, staged = c.staged;
+  int lines = 0, first = 4;
+  for (int m = 2; m >= 0; --m)
+    if (tb[m] >= 1 && tb[m] <= 3) ++lines, first = tb[m];
+  const bool bit0 = tb[0] == 0, one_two = tb[0] == 1 && tb[1] == 2;
+  if (c.es == 4) {
+    // 1 2 3 0.50..0.76; others without bit 0 0.91 up to 2^19, from there up to 1.36;
+    // with it 1.06..1.53; beyond the cache two on lines 0.75, 1 4 6 0.80
+    if (lines == 3) return !staged || c.from(18);
+    if (staged) return false;
+    if (c.beyond()) return lines == 2 || (near && (bit0 ? per : first == 1));
+    return !bit0 && c.up_to(19) && (lines == 2 || (near && (!per || first < 4)));
+  }
+  if (c.es == 8) {
+    if (bit0) {
+      // 0 1 2 61 -> 52 (1.03 below 2^20); others 1.05..1.15 with one operator
+      if (tb[2] == 2) return per ? !staged || c.from(21) : c.from(20);
+      return near && per && !staged && c.from(20);
+    }
+    // 1 2 3 79 -> 50, h 1 2 64 -> 50; staged 1.10 below 2^19 and 1.20 below 2^20
+    if (lines == 3) return !staged || c.from(19);
+    if (one_two) return !staged || c.from(20);
+    // h 1 3, h 2 3: 0.74..0.87 up to 2^20, 0.72..0.95 from 2^24, 1.03 between
+    if (lines == 2) return staged ? c.beyond() : per || c.up_to(20) || c.from(24);
+    // 4 5 6: 0.81..0.94 up to 2^20, 0.90 beyond the cache, 1.04..1.13 between
+    if (staged || !near) return false;
+    return per ? first < 3 || (first == 3 && c.from(21)) : c.up_to(20) || c.beyond();
+  }
+  if (bit0) {
+    // 0 1 2 0.57..0.78, 0 1 5 0.64..0.84, h 0 1 0.66..0.93; 0 3 6 0.78 up to 2^19,
+    // 1.09 above; h 0 2 0.79..0.95 up to 2^20, 0.80 from 2^24, 1.18 between
+    if (tb[2] == 2) return !staged || c.from(19);
+    if (tb[1] == 1) return !staged || (near && c.from(20));
+    if (staged) return false;
+    if (!near) return tb[1] == 2 && (per ? c.from(20) : c.up_to(20) || c.from(24));
+    return per ? c.from(20) : c.up_to(19);
+  }
+  // 1 2 6 0.46..0.68, 1 4 6 0.57..0.85, h 1 3 0.62..0.85; staged 1.14 below 2^19
+  if (first == 1) return one_two || !staged || c.from(near ? 18 : 19);
+  // 2 5 7 0.57..0.96; h 2 3, h 2 6 0.63..0.84 up to 2^20, 0.80 from 2^24, 1.18 between
+  if (first == 2 && near && lines == 1) return !staged || c.from(21);
+  if (staged) return false;
+  if (first == 2) return c.up_to(20) || c.from(per ? 23 : 24);
+  // 4 5 6: 0.63..0.94 up to 2^21, 1.03..1.10 above
+  return near && (per ? first == 3 && (c.up_to(20) || c.from(23)) : c.up_to(21));
+}
+
 }  // namespace
 
 // Complex gates on 6..10 qubits on the matrix cores (wide_mfma.hip).
@@ -358,36 +464,14 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
       }
       return check_launch("dense_xch_kernel");
     }
-    // Targets on low index bits (dense_low_kernel).  Where the line lies (24
-    // qubits, complex64, us by index bits of the targets; vector kernel -> this
-    // one):
-    //   3 targets      0 1 2  61 -> 45, 1 2 3  79 -> 45, 5 6 8  49 -> 44
-    //   2, one of 1..3 1 2    65 -> 42, 2 3    55 -> 41, 0 2    45 -> 42
-    //   2 others       0 5    41 -> 41, 4 6    43 -> 41 (20 qubits 3.6 -> 3.9)
-    // With one operator per state 12 qubits x 4096: 1 2  64 -> 41, 0 5  60 -> 41,
-    // 0 1 2  59 -> 45, but 5 6 8  43 -> 45.  With targets beyond the block two on
-    // bits 1..3 (h the highest bit): h 1 2  64 -> 46, 26 qubits 250 -> 191;
-    // complex128 any: 23 qubits h 1  61 -> 43, h 0 1  62 -> 50; one alone gains
-    // nothing in complex64 (22 qubits h 1  13.9 -> 14.5) and loses in float32
-    // (45 -> 50), but does with one operator per state (h 1  48 -> 42).  A few wavefronts only (under 12
-    // qubits) wait longer for its three trips through LDS: 1.84 -> 1.95.
     if ((k == 2 || k == 3) && io_aligned && n >= k + 6) {
       LowParams l{};
       int near = 0;                  // targets inside the contiguous run
       while (near < k && tb[near] < 6 + near + 1) ++near;
-      int line_bits = 0, lowest = 4; // targets on bits 1..3, the first of them
-      for (int m = k - 1; m >= 0; --m)
-        if (tb[m] >= 1 && tb[m] <= 3) ++line_bits, lowest = tb[m];
-      const int64_t waves = batch << (n - k - 6);
-      bool low;
-      if (near < k)
-        low = near > 0 && (line_bits >= 2 || (es == 16 && lowest < (k == 2 ? 4 : 3)) ||
-                           (op_bstride != 0 && k == 2 && es >= 8 && (line_bits || tb[0] == 0)));
-      else if (k == 3)
-        low = op_bstride == 0 || tb[0] <= 3;
-      else
-        low = line_bits || (op_bstride != 0 && tb[0] == 0);
-      low = low && waves >= (k == 3 ? 64 : 16);
+      LowCase c{es, tb, near, batch << n, op_bstride != 0, false};
+      c.staged = k == 3 && c.per && n - k - (tb[0] == 0 ? 0 : 1) >= 8;
+      const bool low = near > 0 && (batch << (n - k - 6)) >= (k == 3 ? 64 : 16) &&
+                       (k == 2 ? low_pays_2(c) : low_pays_3(c));
       if (low) {
         l.beyond = k - near;
         l.log2_run = 6 + near;

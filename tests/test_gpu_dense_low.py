@@ -89,3 +89,35 @@ def test_4_qubit_gates_on_either_side_of_the_matrix_core_rule(device, n, batch):
                 _lib.ptr(y), _lib.ptr(y), _lib.ptr(opd), _lib.UA_COMPLEX64, n, 4,
                 _lib.int_array(qubits), batch, 2 ** n, 0, _lib.stream_handle(device)), "in place")
             assert torch.equal(y, out)
+
+
+@pytest.mark.parametrize("dt", list(TOL))
+@pytest.mark.parametrize("n,batch,per_state", [(12, 64, True), (12, 300, True), (12, 2048, True),
+                                               (10, 1024, True), (10, 4097, True),
+                                               (18, 1, False), (19, 1, False), (20, 1, False),
+                                               (13, 300, False), (24, 1, False)])
+def test_low_targets_on_either_side_of_the_sizes(device, dt, n, batch, per_state):
+    """From states that wait for accesses to states beyond the caches: whichever
+    kernel the size calls for, the bits are those of the general one (the same
+    call on a state one element off the alignment)."""
+    g = torch.Generator(device=device).manual_seed(n + batch)
+    size = batch * 2 ** n
+    buf = torch.empty(2 * size + 4, dtype=dt, device=device)
+    off, res = buf[1:1 + size].view(batch, 2 ** n), buf[size + 1:2 * size + 1].view(batch, -1)
+    x = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=dt)
+    off.copy_(x)
+    for k in (2, 3):
+        ops = torch.randn(((batch,) if per_state else ()) + (2 ** k, 2 ** k), generator=g,
+                          device=device, dtype=dt)
+        for bits in BITS[k] + [(0, 3), (3, 5), (n - 1, 0)][:3 * (3 - k)] + \
+                [(n - 1, 1, 3), (n - 1, 0, 2), (6, 7, 8)][:3 * (k - 2)]:
+            if max(bits) >= n:
+                continue
+            qubits = _lib.int_array([n - 1 - b for b in bits])
+            for o, i in ((res, off), (x, x.clone())):
+                _lib.check(_lib.load().ua_apply_operator(
+                    _lib.ptr(o), _lib.ptr(i), _lib.ptr(ops), _lib.DTYPE_CODES[dt], n, k, qubits,
+                    batch, 2 ** n, 4 ** k if per_state else 0, _lib.stream_handle(device)),
+                    "apply_operator")
+            assert torch.equal(res, x), bits
+            x.copy_(off)
