@@ -434,11 +434,13 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
     // speed: 26 qubits 208..225 us, matrix cores 222..235) or the states stay
     // in the caches, where the vector kernel waits for LDS and the matrix: 16
     // qubits 8.6..12.9 -> 3.0 us, 22 qubits 16.6..20 -> 14.5..16.8 (23 qubits
-    // with several states in turn: 28..40 and 26..45, by the targets).
+    // with several states in turn: 28..40 and 26..45, by the targets).  With a
+    // target on bit 0, which the vector kernel pairs, the line is 2^21 amplitudes
+    // (22 qubits 16.8 and 18.2).
     const bool mfma_shape =
         (k == 5 && dtype != UA_FLOAT32 && dtype != UA_FLOAT64) ||
         (k == 4 && dtype == UA_COMPLEX128) || (k == 4 && dtype == UA_COMPLEX64 &&
-         (tb[k - 1] < 6 || batch <= ((int64_t(1) << 22) >> n)));
+         (tb[k - 1] < 6 || batch <= ((int64_t(1) << (tb[0] == 0 ? 21 : 22)) >> n)));
     if (g_use_mfma && mfma_shape && op_bstride == 0 && n - k >= 6)
       return apply_dense_mfma(out, state, op, dtype, n, k, tb, gp, batch, state_bstride, s);
 

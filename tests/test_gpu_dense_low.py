@@ -121,3 +121,20 @@ def test_low_targets_on_either_side_of_the_sizes(device, dt, n, batch, per_state
                     "apply_operator")
             assert torch.equal(res, x), bits
             x.copy_(off)
+
+
+@pytest.mark.parametrize("batch", [256, 257, 512])
+def test_4_qubit_gates_on_the_lowest_bit(device, batch):
+    """complex64 states of 13 qubits around 2^21 and 2^22 amplitudes in all, where gates
+    with and without a target on the lowest bit change kernels."""
+    n = 13
+    g = torch.Generator(device=device).manual_seed(batch)
+    x = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=torch.complex64)
+    op = torch.randn(16, 16, generator=g, device=device, dtype=torch.complex64)
+    pick = [0, batch // 2, batch - 1]
+    for bits in [(0, 5, 9, 12), (7, 0, 6, 8), (1, 5, 9, 12)]:
+        qubits = [n - 1 - b for b in bits]
+        out = sim.apply_operator(op, qubits, x)
+        ref = U.apply_operator(op.cpu().numpy().astype(np.complex128), qubits,
+                               x[pick].cpu().numpy().astype(np.complex128))
+        assert np.max(np.abs(out[pick].cpu().numpy() - ref)) / np.max(np.abs(ref)) < 8e-6, bits
