@@ -6,6 +6,8 @@
 // reads each amplitude and each angle once, forms cos/sin in registers and
 // writes the product.  `out` may equal `state` (in place) when both are
 // contiguous with the output's shape.
+#include <type_traits>
+
 #include "ua_common.h"
 
 namespace ua {
@@ -182,21 +184,33 @@ void launch_phase(int mode, void* out, const void* st, const void* an,
     phase_pair_kernel<TO, TS, TA, 2><<<grid_for(pairs, kBlock * 2), kBlock, 0, s>>>(o, x, a, pairs);
     return;
   }
-  // Rows that fill the 64 lanes of a row group at least
+  // phase_rows_kernel from 2^18 amplitudes (complex64: 1024 x 301 0.93 of the time
+  // of the loop over elements, 65536 x 64 0.78; 1024 x 64 1.10, which waits for its
+  // longer chain), where the workgroups along a row are seven eighths full at
+  // least (130 columns, two thirds: 1.2), and not for factors of 32 bits in a
+  // complex128 product (1.00..1.19) or complex128 rows of 4 MB and more with 64 MB
+  // of states (1.03; shorter ones 0.8..0.95).
   constexpr int W = 16 / sizeof(TO);
-  if (mode == TILE && pair_ok && p.tile % W == 0 && p.tile >= 64 * W) {
-    const int64_t rows = p.total / p.tile, groups = p.tile / W;
-    const int tx = groups >= kBlock ? kBlock : 64, ty = kBlock / tx;
-    const int64_t gx = (groups + tx - 1) / tx;
-    int64_t gy = (rows + ty * kRows - 1) / (ty * kRows);
-    if (gy > 65535) gy = 65535;
-    if (gx <= 0x7fffffffLL) {
-      const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
-      if (tx == kBlock)
-        phase_rows_kernel<TO, TS, TA, kBlock><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
-      else
-        phase_rows_kernel<TO, TS, TA, 64><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
-      return;
+  constexpr bool kWideAngles = std::is_same_v<TA, double> || std::is_same_v<TA, double2>;
+  constexpr bool kRowsPay = sizeof(TO) == 8 || kWideAngles;
+  constexpr bool kAllWide = sizeof(TS) == 16 && std::is_same_v<TA, double>;
+  if constexpr (kRowsPay) {
+    if (mode == TILE && pair_ok && p.tile % W == 0 && p.tile >= 64 * W &&
+        p.total >= (int64_t(1) << 18) &&
+        !(kAllWide && p.tile >= (int64_t(1) << 18) && p.total >= (int64_t(1) << 22))) {
+      const int64_t rows = p.total / p.tile, groups = p.tile / W;
+      const int tx = groups >= kBlock ? kBlock : 64, ty = kBlock / tx;
+      const int64_t gx = (groups + tx - 1) / tx;
+      int64_t gy = (rows + ty * kRows - 1) / (ty * kRows);
+      if (gy > 65535) gy = 65535;
+      if (gx <= 0x7fffffffLL && 8 * groups >= 7 * gx * tx) {
+        const dim3 grid(static_cast<unsigned>(gx), static_cast<unsigned>(gy));
+        if (tx == kBlock)
+          phase_rows_kernel<TO, TS, TA, kBlock><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
+        else
+          phase_rows_kernel<TO, TS, TA, 64><<<grid, kBlock, 0, s>>>(o, x, a, p.tile, rows);
+        return;
+      }
     }
   }
   switch (mode) {

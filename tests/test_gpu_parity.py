@@ -509,3 +509,24 @@ def test_qubits_out_of_range_are_refused(device):
             sim.apply_operator(op, bad, st)
     with pytest.raises(TypeError):
         sim.apply_operator(op, [[1]], st)
+
+
+@pytest.mark.parametrize("at,dt", [(torch.float32, torch.complex64),
+                                   (torch.float64, torch.complex128),
+                                   (torch.float32, torch.complex128),
+                                   (torch.float64, torch.complex64),
+                                   (torch.complex128, torch.complex128)])
+@pytest.mark.parametrize("cols,rows", [(128, 2047), (128, 2048), (130, 2100), (448, 601), (446, 601),
+                                       (2 ** 18, 15), (2 ** 18, 16)])
+def test_apply_phase_on_either_side_of_the_row_kernel(device, at, dt, cols, rows):
+    """Just under and at its least size, rows that fill their workgroups well and
+    badly, long complex128 rows: factors rounded once, products three times more."""
+    g = torch.Generator(device=device).manual_seed(cols + rows)
+    a = torch.randn(cols, generator=g, device=device, dtype=at)
+    if at.is_complex:
+        a = a.real + 0.1j * a.imag
+    x = torch.randn(rows, cols, generator=g, device=device, dtype=dt)
+    out = sim.apply_phase(a, x)
+    ref = torch.exp(-1j * a.to(torch.complex128)) * x.to(torch.complex128)
+    eps = 2.0 ** -24 if torch.float32 in (at, dt) or torch.complex64 in (at, dt) else 2.0 ** -53
+    assert float(((out - ref).abs() / ref.abs()).max()) < 16 * eps
