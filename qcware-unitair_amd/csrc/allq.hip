@@ -145,9 +145,12 @@ struct AllqPass {
   int stage_apply[kMaxStages];     // 4-bit mask: cube bits that get a gate
   int stage_slot[kMaxStages][4];   // target index of each cube bit's gate
   int num_stages;
+  int staged;                // one stage that meets the state through LDS
 };
 
-template <typename T, int TB>
+// STAGED: the one stage's cubes would split the lines of memory (plan_layer), so
+// the tile moves in whole lines and LDS lies on both sides of the stage.
+template <typename T, int TB, bool STAGED>
 __global__ __launch_bounds__((1 << TB) / kCube) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 2)))
 void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a) {
   constexpr int kTile = 1 << TB;
@@ -164,12 +167,32 @@ void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a)
   const int64_t origin = int64_t(insert_zero_bits(
       uint64_t(tg) & ((uint64_t(1) << a.log2_tiles) - 1), a.local, TB));
   const T* ops_b = op + b * a.op_bstride;
-  for (int st = 0; st < a.num_stages; ++st) {
+  constexpr int kThreads = kTile / kCube;
+  int64_t dep_t = 0, dep_k[STAGED ? 8 : 1];
+  if constexpr (STAGED) {
+    // element pair e = 2 * tid + 2 * kThreads * k, tile bit i = state bit local[i]
+#pragma unroll
+    for (int i = 1; i <= TB - 4; ++i) dep_t |= int64_t(((2 * tid) >> i) & 1) << a.local[i];
+    const T* src = in + b * a.in_bstride + origin + dep_t;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      dep_k[k] = 0;
+#pragma unroll
+      for (int i = TB - 3; i < TB; ++i)
+        dep_k[k] |= int64_t((k >> (i - (TB - 3))) & 1) << a.local[i];
+      T v0, v1;
+      load_pair(src + dep_k[k], v0, v1);
+      const int e = 2 * tid + 2 * kThreads * k;
+      tile[lds_pos(e)] = v0;
+      tile[lds_pos(e + 1)] = v1;
+    }
+  }
+  for (int st = 0; st < (STAGED ? 1 : a.num_stages); ++st) {
     const int sb[4] = {a.stage_bits[st][0], a.stage_bits[st][1], a.stage_bits[st][2],
                        a.stage_bits[st][3]};
     const int e0 = int(insert_zero_bits(uint64_t(tid), sb, 4));
     const int m0 = 1 << sb[0], m1 = 1 << sb[1], m2 = 1 << sb[2], m3 = 1 << sb[3];
-    const bool first = st == 0, last = st == a.num_stages - 1;
+    const bool first = !STAGED && st == 0, last = !STAGED && st == a.num_stages - 1;
     // the first and the last stage hold tile bit 0 (= state bit 0): their
     // cubes are 8 pairs of adjacent amplitudes, read from and written to the
     // state without a trip through LDS
@@ -223,6 +246,15 @@ void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a)
       }
     }
   }
+  if constexpr (STAGED) {
+    __syncthreads();
+    T* dst = out + b * N + origin + dep_t;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int e = 2 * tid + 2 * kThreads * k;
+      store_pair(dst + dep_k[k], tile[lds_pos(e)], tile[lds_pos(e + 1)]);
+    }
+  }
 }
 
 // Plan the passes for the gates on the state bits in `active` (slot[bit] =
@@ -233,7 +265,9 @@ void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a)
 // last stage padded with bits that carry no gate there).  With no target at
 // all, one pass without stages copies the input.  Returns the number of
 // passes (at most 8; needs R < TB <= n).
-int plan_layer(int n, uint64_t active, const int* slot, int TB, int R, AllqPass* passes) {
+int plan_layer(int n, uint64_t active, const int* slot, int TB, int R, int64_t amps,
+               AllqPass* passes) {
+  const bool c64 = R == 2;
   const uint64_t low_mask = (uint64_t(1) << R) - 1;
   int rest[64], nrest = 0;
   for (int bit = R; bit < n; ++bit)
@@ -260,22 +294,53 @@ int plan_layer(int n, uint64_t active, const int* slot, int TB, int R, AllqPass*
     const bool gate0 = ng > 0 && pos_of_gate[0] == 0;
     int others[kMaxTileBits], no = 0;  // gates above tile bit 0, descending
     for (int g = ng - 1; g >= (gate0 ? 1 : 0); --g) others[no++] = pos_of_gate[g];
-    p.num_stages = no <= 3 ? 1 : 2 + (no > 6 ? (no - 6 + 3) / 4 : 0);
-    int taken = 0;
+    // A direct stage with gates inside a 128-byte line leaves the lanes parts of
+    // lines.  Small states do not mind (complex64 12 qubits, gate on bit 1: 3.6 us
+    // through LDS, 3.0 direct), from 8 (complex128: 4) MB they do (22 qubits 12.0
+    // and 14.5, bits 1 and 2 12.6 and 19.2, 24 qubits 42.5 and 59), three such bits
+    // (complex128: bits 1 and 2) at any size.  Up to four gates then move through
+    // LDS on both sides; of more, those go to the stages in between (complex64 bits
+    // 0..5 at 24 qubits: 62 direct, 45 so).  (complex64's bit 3 alone costs nothing.)
+    const int taken_first = no < 3 ? no : 3, between4 = no > 6 ? (no - 3) / 4 * 4 : 0;
+    const int taken_last = no - taken_first > between4 ? no - taken_first - between4 : 0;
+    int lines = 0, worst = 0;          // bits 1 and 2; all bits of a line in one end
+    auto count = [&](int from, int to) {
+      int w = 0;
+      for (int i = from; i < to; ++i) {
+        const int bit = p.local[others[i]];
+        lines += bit < 3 && (c64 || bit == 1);
+        w += bit < R + 2;
+      }
+      if (w > worst) worst = w;
+    };
+    count(0, taken_first);
+    count(no - taken_last, no);
+    const bool spread = (lines && amps >= (int64_t(1) << (c64 ? 20 : 18))) ||
+                        worst >= (c64 ? 3 : 2) || (!c64 && lines && ng == 4 && !gate0);
+    p.staged = spread && ng <= 4;
+    int ends[kMaxTileBits], ne = 0, mids[kMaxTileBits], nm = 0;
+    for (int i = 0; i < no; ++i) {
+      const bool mid = spread ? p.local[others[i]] < R + 2 || ne == 6
+                              : i >= taken_first && i < no - taken_last;
+      if (mid) mids[nm++] = others[i];
+      else ends[ne++] = others[i];
+    }
+    p.num_stages = nm == 0 && ne <= 3 ? 1 : 2 + (nm + 3) / 4;
+    if (p.staged) {
+      p.num_stages = 1;
+      nm = 0;
+      for (ne = 0; ne < no; ++ne) ends[ne] = others[ne];
+    }
+    int taken = 0, between = 0;
     for (int st = 0; st < p.num_stages; ++st) {
       const bool first = st == 0, end = first || st == p.num_stages - 1;
       int cube[4], on[4], nc = 0;
-      if (end) {
+      if (end && !(p.staged && !gate0)) {
         cube[nc] = 0;
         on[nc++] = first && gate0;
       }
-      // the last stage takes what is left, at most three
-      const int left = no - taken, later = p.num_stages - 1 - st;
-      int take = end ? 3 : 4;
-      if (later == 0) take = left;
-      else if (take > left) take = left;
-      for (int i = 0; i < take; ++i) {
-        cube[nc] = others[taken++];
+      while (nc < 4 && (end ? taken < ne : between < nm)) {
+        cube[nc] = end ? ends[taken++] : mids[between++];
         on[nc++] = 1;
       }
       for (int t = TB - 1; nc < 4; --t) {  // pad with tile bits outside this cube
@@ -349,10 +414,10 @@ int layer_impl(void* out, const void* state, const void* op, int dtype, int n,
     const int line_bits = c64 ? 4 : 3;  // 128-byte lines
     AllqPass passes[8];
     int TB = kMinTileBits;
-    int np = plan_layer(n, active, slot, TB, R, passes);
+    int np = plan_layer(n, active, slot, TB, R, batch << n, passes);
     if (c64 && n >= kMaxTileBits) {
       AllqPass wide[8];
-      const int np13 = plan_layer(n, active, slot, kMaxTileBits, R, wide);
+      const int np13 = plan_layer(n, active, slot, kMaxTileBits, R, batch << n, wide);
       if (np13 < np) {
         TB = kMaxTileBits;
         np = np13;
@@ -380,18 +445,21 @@ int layer_impl(void* out, const void* state, const void* op, int dtype, int n,
       p.xcd_order = shares && p.total_tiles % 8 == 0;
       const void* src = (i == 0) ? state : out;
       const unsigned grid = unsigned(p.total_tiles);
-      if (TB == kMaxTileBits)
-        allq_pass_kernel<float2, 13><<<grid, (1 << 13) / kCube, 0, s>>>(
-            static_cast<float2*>(out), static_cast<const float2*>(src),
-            static_cast<const float2*>(op), p);
-      else if (c64)
-        allq_pass_kernel<float2, 12><<<grid, (1 << 12) / kCube, 0, s>>>(
-            static_cast<float2*>(out), static_cast<const float2*>(src),
-            static_cast<const float2*>(op), p);
-      else
-        allq_pass_kernel<double2, 12><<<grid, (1 << 12) / kCube, 0, s>>>(
-            static_cast<double2*>(out), static_cast<const double2*>(src),
-            static_cast<const double2*>(op), p);
+#define UA_ALLQ(TT, BITS)                                                              \
+      do {                                                                             \
+        if (p.staged)                                                                  \
+          allq_pass_kernel<TT, BITS, true><<<grid, (1 << BITS) / kCube, 0, s>>>(       \
+              static_cast<TT*>(out), static_cast<const TT*>(src),                      \
+              static_cast<const TT*>(op), p);                                          \
+        else                                                                           \
+          allq_pass_kernel<TT, BITS, false><<<grid, (1 << BITS) / kCube, 0, s>>>(      \
+              static_cast<TT*>(out), static_cast<const TT*>(src),                      \
+              static_cast<const TT*>(op), p);                                          \
+      } while (0)
+      if (TB == kMaxTileBits) UA_ALLQ(float2, 13);
+      else if (c64) UA_ALLQ(float2, 12);
+      else UA_ALLQ(double2, 12);
+#undef UA_ALLQ
       const int rc = check_launch("allq_pass_kernel");
       if (rc) return rc;
     }

@@ -243,3 +243,22 @@ def test_layer_stage_counts(device, dt, count, with_bit0):
     ref = U.apply_to_qubits([o.astype(np.complex128) for o in ops], qubits,
                             st.astype(np.complex128))
     assert rel(out.cpu().numpy(), ref) < TOL[dt] * count
+
+
+@pytest.mark.parametrize("dt,n,batch", [(torch.complex64, 12, 3), (torch.complex64, 20, 1),
+                                        (torch.complex128, 12, 3), (torch.complex128, 18, 1)])
+@pytest.mark.parametrize("bits", [(1,), (2,), (0, 1), (1, 2), (2, 3), (1, 2, 3), (0, 1, 2, 3),
+                                  (1, 5, 8, 10), (1, 2, 8, 10), (0, 1, 2, 3, 4), (0, 1, 2, 3, 4, 5),
+                                  (1, 3, 5, 7, 9, 11), tuple(range(12))])
+def test_layer_gates_inside_a_line(device, dt, n, batch, bits):
+    """Gates on the index bits of a 128-byte line, at sizes that move their cubes
+    directly, through LDS on both sides, or between other stages."""
+    rng = np.random.default_rng(n + len(bits))
+    qubits = [n - 1 - b for b in rng.permutation(bits)]
+    ops = [cast(rand((2, 2), dt, rng), dt) for _ in qubits]
+    st = cast(rand((batch, 2 ** n), dt, rng), dt)
+    out = sim.apply_to_qubits([torch.from_numpy(o).to(device) for o in ops], qubits,
+                              torch.from_numpy(st).to(device))
+    ref = U.apply_to_qubits([o.astype(np.complex128) for o in ops], qubits,
+                            st.astype(np.complex128))
+    assert rel(out.cpu().numpy(), ref) < TOL[dt] * len(bits)
