@@ -67,12 +67,13 @@ __host__ __device__ __forceinline__ constexpr int gemm_pos(int c, int g) {
 }
 
 // RTW: row tiles of 16 per wavefront.  WR wavefronts (WR_, or as many as there
-// are row tiles for) cover the rows of a workgroup, WC the groups.
-template <typename T, int K, int LG, int RTW, int WR_ = 0> struct GemmShape {
+// are row tiles for) cover the rows of a workgroup, WC the groups, KS ranges of
+// the columns.
+template <typename T, int K, int LG, int RTW, int WR_ = 0, int KS = 1> struct GemmShape {
   static constexpr int D = 1 << K, G = 1 << LG, TB = K + LG;
   static constexpr int RT = D / 16, CT = G / 16;
   static constexpr int WR = WR_ ? WR_ : RT / RTW < kWaves ? RT / RTW : kWaves;
-  static constexpr int WC = kWaves / WR;
+  static constexpr int WC = kWaves / WR / KS;
   static constexpr int CTW = CT / WC;
   static constexpr int S = RT / (WR * RTW);   // row slices (blockIdx.y)
   static constexpr int AC = 32 / sizeof(T);   // columns of U a lane reads a step: 32 bytes
@@ -82,14 +83,15 @@ template <typename T, int K, int LG, int RTW, int WR_ = 0> struct GemmShape {
   // 8-qubit complex64 gates sum 512 real terms as four partial sums of 128 (error
   // of a random gate 2.1e-7; 4.1e-7 in one chain)
   static constexpr int NSUM = K == 8 && sizeof(T) == 8 ? 4 : 1;
-  static_assert(WR * WC == kWaves && CTW * WC == CT && S * WR * RTW == RT, "split");
+  static_assert(WR * WC * KS == kWaves && CTW * WC == CT && S * WR * RTW == RT, "split");
+  static_assert(KS == 1 || (KS == NSUM && S > 1), "a wavefront's columns are a partial sum");
 };
 
-template <typename T, int K, int LG, int RTW, int WR_ = 0>
+template <typename T, int K, int LG, int RTW, int WR_ = 0, int KS = 1>
 __global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(2 * GemmShape<T, K, LG, RTW, WR_>::kPerCu)))
+__attribute__((amdgpu_waves_per_eu(2 * GemmShape<T, K, LG, RTW, WR_, KS>::kPerCu)))
 void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
-  using Sh = GemmShape<T, K, LG, RTW, WR_>;
+  using Sh = GemmShape<T, K, LG, RTW, WR_, KS>;
   using R = typename RealOf<T>::type;
   using M = Mfma<R>;
   constexpr int D = Sh::D, TB = Sh::TB, CTW = Sh::CTW;
@@ -107,7 +109,9 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
   const T* U = static_cast<const T*>(p.op) + b * p.op_bstride;
 
   // ---- this wavefront's row and group tiles; its first columns of U
-  const int wr = wave % Sh::WR, wc = wave / Sh::WR;
+  const int wr = wave % Sh::WR, wc = wave / Sh::WR % Sh::WC, ks = wave / Sh::WR / Sh::WC;
+  constexpr int KW = KK / KS;            // steps of a wavefront, from kb on
+  const int kb = ks * KW;
   const int t0 = (int(blockIdx.y) * Sh::WR + wr) * RTW;
   const int g0 = 16 * CTW * wc;
   const T* urow = U + int64_t(16 * t0 + l16) * D + AC * q;
@@ -123,7 +127,7 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
         dst[i][2 * h + 1] = v.v[1];
       }
   };
-  load_a(a, 0);
+  load_a(a, kb);
 
   // ---- the tile: element pair e = 2 * (tid + kThreads * u), tile bit i = state bit local[i]
   int64_t dep_t = 0;
@@ -193,7 +197,7 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
   static_assert(KK % (2 * Sh::NSUM) == 0, "two steps a turn");
   T a1[RTW][AC];
 #pragma unroll 1
-  for (int k0 = 0; k0 < KK; k0 += KK / Sh::NSUM) {
+  for (int k0 = kb; k0 < kb + KW; k0 += KK / Sh::NSUM) {
 #pragma unroll 1
     for (int kk = k0; kk < k0 + KK / Sh::NSUM; kk += 2) {
       // each step's columns are requested a step ahead; the scheduler would
@@ -201,11 +205,11 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
       load_a(a1, kk + 1);
       __builtin_amdgcn_sched_barrier(0);
       step(a, kk);
-      load_a(a, kk + 2 < KK ? kk + 2 : kk);
+      load_a(a, kk + 2 < kb + KW ? kk + 2 : kk);
       __builtin_amdgcn_sched_barrier(0);
       step(a1, kk + 1);
     }
-    if constexpr (Sh::NSUM > 1) {  // a partial sum is complete
+    if constexpr (Sh::NSUM > 1 && KS == 1) {  // a partial sum is complete
       const bool start = k0 == 0, end = k0 + KK / Sh::NSUM == KK;
 #pragma unroll
       for (int i = 0; i < RTW; ++i)
@@ -220,6 +224,38 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
   }
 
   T* dst = out + b * p.bstride + origin;
+  if constexpr (KS > 1) {
+    // ---- the wavefronts' partial sums meet in LDS, in the order of one chain
+    constexpr int PART = RTW * CTW * 4 * 64;
+    static_assert(Sh::WR * Sh::WC * KS * PART <= (1 << TB), "the tile's place holds them");
+    T* const mine = xs + wave * PART + lane;
+    __syncthreads();  // every input is read
+#pragma unroll
+    for (int i = 0; i < RTW; ++i)
+#pragma unroll
+      for (int c = 0; c < CTW; ++c)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          T v;
+          v.x = re[i][c][r];
+          v.y = im[i][c][r];
+          mine[((i * CTW + c) * 4 + r) * 64] = v;
+        }
+    __syncthreads();
+    if (ks > 0) return;  // no barrier follows
+#pragma unroll
+    for (int k = 1; k < KS; ++k)
+#pragma unroll
+      for (int i = 0; i < RTW; ++i)
+#pragma unroll
+        for (int c = 0; c < CTW; ++c)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const T v = mine[k * Sh::WR * Sh::WC * PART + ((i * CTW + c) * 4 + r) * 64];
+            re[i][c][r] += v.x;
+            im[i][c][r] += v.y;
+          }
+  }
   if constexpr (Sh::S > 1) {
     // ---- a slice of the rows, straight from the accumulators
     int64_t lane_off = 0;
@@ -282,9 +318,9 @@ struct GemmArgs {
   hipStream_t s;
 };
 
-template <typename T, int K, int LG, int RTW, int WR_ = 0>
+template <typename T, int K, int LG, int RTW, int WR_ = 0, int KS = 1>
 int launch_gemm(const GemmArgs& a) {
-  using Sh = GemmShape<T, K, LG, RTW, WR_>;
+  using Sh = GemmShape<T, K, LG, RTW, WR_, KS>;
   GemmPass p{};
   p.op = a.op;
   p.log2_tiles = a.n - Sh::TB;
@@ -315,7 +351,7 @@ int launch_gemm(const GemmArgs& a) {
     for (int j = 0; j < LG; ++j)
       if (p.gbit[j] == bit) p.pcol[i] = gemm_pos<T, LG>(0, 1 << j);
   }
-  dense_gemm_kernel<T, K, LG, RTW, WR_><<<dim3(unsigned(p.tiles), Sh::S), kThreads, 0, a.s>>>(
+  dense_gemm_kernel<T, K, LG, RTW, WR_, KS><<<dim3(unsigned(p.tiles), Sh::S), kThreads, 0, a.s>>>(
       static_cast<T*>(a.out), static_cast<const T*>(a.in), p);
   return check_launch("dense_gemm_kernel");
 }
@@ -367,7 +403,18 @@ int apply_dense_gemm(void* out, const void* in, const void* op, int dtype, int n
   if (dtype == UA_COMPLEX64) switch (k) {
     case 6: return split ? launch_gemm<float2, 6, 6, 1, 2>(a) : launch_gemm<float2, 6, 6, 1>(a);
     case 7: return split ? launch_gemm<float2, 7, 5, 1, 4>(a) : launch_gemm<float2, 7, 5, 1>(a);
-    case 8: return split ? launch_gemm<float2, 8, 5, 1, 4>(a) : launch_gemm<float2, 8, 5, 2>(a);
+    case 8:
+      // Few tiles: the wavefronts of a workgroup split the columns too (the partial
+      // sums are there anyway), and the rows of a tile go to 16 workgroups or to
+      // 8 (14 qubits, 2 tiles 5.6 and 8.2 us, in rows alone 14; 32 tiles 8.9 and
+      // 9.0, 64 tiles 13.8 and 12.0, 224 tiles 51 and 43, 40 in one piece).  Little more
+      // than 256 tiles leave a second round nearly empty: 320 tiles 78 us in one
+      // piece, 66 so; from 384 on one piece is faster (78 and 79).
+      if (disjoint(a, 8) && (tiles <= 352 && tiles != 256)) {
+        if (tiles <= 48) return launch_gemm<float2, 8, 5, 1, 1, 4>(a);
+        return launch_gemm<float2, 8, 5, 1, 2, 4>(a);
+      }
+      return launch_gemm<float2, 8, 5, 2>(a);
     case 9: return split ? launch_gemm<float2, 9, 5, 1, 4>(a) : launch_gemm<float2, 9, 5, 4>(a);
     default: return split ? launch_gemm<float2, 10, 4, 1>(a) : launch_gemm<float2, 10, 4, 8>(a);
   }

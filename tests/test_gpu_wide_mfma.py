@@ -71,3 +71,30 @@ def test_wide_gates_many_tiles(device, dt, k, n):
                              torch.from_numpy(st).to(device))
     ref = U.apply_operator(op.astype(np.complex128), qubits, st.astype(np.complex128))
     assert _rel(out.cpu().numpy(), ref) < TOL[dt]
+
+
+# 2, 48, 50, 254, 256, 320, 352 and 354 tiles of 2^13 amplitudes
+@pytest.mark.parametrize("n,batch", [(14, 1), (14, 24), (14, 25), (14, 127), (14, 128), (15, 80),
+                                     (14, 176), (14, 177)])
+def test_8_qubit_gates_by_tiles(device, n, batch):
+    """complex64: columns split over the wavefronts and rows over 16 or 8
+    workgroups of a tile, or a tile in one piece; in place (one operator for each
+    entry: in one piece) the sums are the same, in the same order."""
+    k = 8
+    rng = np.random.default_rng(batch)
+    g = torch.Generator(device=device).manual_seed(batch)
+    st = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=torch.complex64)
+    op = _rand((2 ** k, 2 ** k), rng, torch.complex64) / np.complex64(16)
+    opd = torch.from_numpy(op).to(device)
+    pick = sorted({0, batch // 2, batch - 1})
+    for bits in (list(range(k)), [int(b) for b in rng.permutation(n)[:k]]):
+        qubits = [n - 1 - b for b in bits]
+        out = sim.apply_operator(opd, qubits, st)
+        ref = U.apply_operator(op.astype(np.complex128), qubits,
+                               st[pick].cpu().numpy().astype(np.complex128))
+        assert _rel(out[pick].cpu().numpy(), ref) < TOL[torch.complex64]
+        x, ops = st.clone(), opd.expand(batch, -1, -1).contiguous()
+        _lib.check(_lib.load().ua_apply_operator(
+            _lib.ptr(x), _lib.ptr(x), _lib.ptr(ops), _lib.UA_COMPLEX64, n, k,
+            _lib.int_array(qubits), batch, 2 ** n, 4 ** k, _lib.stream_handle(device)), "in place")
+        assert torch.equal(x, out)
