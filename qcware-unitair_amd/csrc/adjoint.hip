@@ -1068,6 +1068,27 @@ struct OpGradShape {
   int64_t nblk, parts, units, units_per_part;
 };
 
+// Complex operators on 4 qubits and complex64 ones on 5: whether the matrix cores
+// (op_grad_mfma_kernel) are faster than the 4 x 4 blocks.  They are where one
+// workgroup does an operator (up to 128 groups of 4 qubits, 64 of 5; 256 operators
+// of 64 groups 71 -> 4 and 272 -> 8 us) and where the groups are many (5 qubits,
+// 4096: 17.5 -> 13.2); between, several operators wait for their parts' whole
+// results to be written and added (16 of 4 qubits, 256 groups each: 9.2 -> 10.7 in
+// complex64, 9.1 -> 12.7 in complex128; one of 5, 512 groups: 9.8 -> 12.8).  With
+// low targets, which the blocks read worst, the line lies lower (16 of 4 qubits,
+// 1024 groups: complex64 13.7 -> 11.7, complex128 19.7 -> 12.6; one of 5, 2048:
+// 16.5 -> 13.3).  sorted: ascending target bits; groups: of one operator.
+bool op_grad_on_mfma(int dtype, int k, const int* sorted, int64_t groups, int64_t op_count) {
+  const bool c64 = dtype == UA_COMPLEX64, several = op_count >= 8;
+  const bool low = c64 ? sorted[k - 1] < 6 : sorted[0] == 0;
+  if (k == 4 && (c64 || dtype == UA_COMPLEX128))
+    return !several || groups <= 128 || groups >= (c64 ? 2048 : 4096) || (low && groups >= 1024);
+  if (k == 5 && c64)
+    return groups <= (several ? 128 : 64) || groups >= 4096 ||
+           (low && groups >= (several ? 1024 : 2048));
+  return false;
+}
+
 OpGradShape op_grad_shape(int n, int k, int64_t batch, int64_t op_count, bool mfma) {
   OpGradShape sh{};
   const int64_t D = int64_t(1) << k;
@@ -1166,8 +1187,9 @@ int operator_gradient(void* grad_op, void* grad_state, const void* grad_out, con
   }
   for (int b = 0, m = 0; b < n; ++b)
     if ((seen >> b) & 1) p.sorted[m++] = b;
-  const bool mfma = (k == 4 && (dtype == UA_COMPLEX64 || dtype == UA_COMPLEX128)) ||
-                    (k == 5 && dtype == UA_COMPLEX64);
+  const bool mfma = op_grad_on_mfma(dtype, k, p.sorted,
+                                    op_count == 1 ? batch << (n - k) : int64_t(1) << (n - k),
+                                    op_count);
   const OpGradShape sh = op_grad_shape(n, k, batch, op_count, mfma);
   p.parts = sh.parts;
   p.units = sh.units;

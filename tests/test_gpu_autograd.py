@@ -364,3 +364,25 @@ def test_gradients_that_arrive_lazily_conjugated(device, ob, sb, qubits, wrt):
     ref = grads(lambda o, s: T.apply_operator(o, qubits, s), "cpu")
     for r, g in zip(ref, grads(lambda o, s: sim.apply_operator(o, qubits, s), device)):
         assert torch.allclose(r, g, atol=1e-10)
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("k,n,ob", [(5, 11, 1), (5, 12, 1), (5, 16, 1), (5, 17, 1), (5, 12, 8),
+                                    (5, 13, 8), (5, 15, 8), (4, 11, 8), (4, 12, 8), (4, 14, 8),
+                                    (4, 15, 8), (4, 16, 8), (4, 12, 7)])
+def test_operator_gradient_on_either_side_of_the_matrix_cores(device, dt, k, n, ob):
+    """Group counts around those from which one operator or several take the
+    matrix cores, targets on the lowest and on the highest bits."""
+    torch.manual_seed(n + ob)
+    eps = torch.finfo(torch.float32 if dt == torch.complex64 else torch.float64).eps
+    for bits in (list(range(k)), list(range(n - k, n)), [0, n - 1, 3, n - 3, 5][:k]):
+        qubits = [n - 1 - b for b in bits]
+        op = torch.randn(*([ob] if ob > 1 else []), 2 ** k, 2 ** k, dtype=dt)
+        st = torch.randn(*([ob] if ob > 1 else []), 2 ** n, dtype=dt)
+        ref = _grads_cpu(lambda o, s: T.apply_operator(o, qubits, s),
+                         op.to(torch.complex128), st.to(torch.complex128))
+        got = _grads_gpu(lambda o, s: sim.apply_operator(o, qubits, s), device, op, st)
+        # as above: the incoming gradient depends on the rounded output
+        for r, g in zip(ref, got):
+            scale = float(r.abs().max())
+            assert float((r - g.to(torch.complex128)).abs().max()) <= 2 ** (k + 3) * eps * scale
