@@ -170,3 +170,20 @@ def test_blocks_misaligned_matrix_runs_gate_by_gate(device):
     ref = oc.run_closed_form(circ.gates, psi)
     fe, ma = BAR[torch.complex64]
     assert U.fidelity_error(ref, got) < fe and U.max_abs_error(ref, got) < ma
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n,batch", [(15, 1), (15, 3), (20, 1), (14, 192)])
+def test_blocks_walk_every_tile_either_way(device, dt, n, batch):
+    """Passes that walk the tiles forwards and backwards, 8, 24 and 256 tiles and
+    groups of 256 beyond: against the gates one by one."""
+    rng = np.random.default_rng(n)
+    gates = [Gate("dense", tuple(int(q) for q in rng.choice(n, 5, replace=False)),
+                  matrix=haar_unitary(32, rng)) for _ in range(7)]
+    g = torch.Generator(device=device).manual_seed(n)
+    x = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=dt) / 2 ** (n / 2)
+    a, b = (CircuitRunner(Circuit(n, gates), dtype=dt, device=device, in_place=True,
+                          dense_blocks=blocks).run(x.clone()) for blocks in (True, False))
+    # 7 gates of 64 real products each
+    eps = 2.0 ** -24 if dt == torch.complex64 else 2.0 ** -53
+    assert float((a - b).abs().max()) < 7 * 64 * eps * float(x.abs().max())
