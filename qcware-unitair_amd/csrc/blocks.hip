@@ -357,6 +357,16 @@ int check_gates(int n, const ua_gate* gates, int num_gates) {
   return UA_OK;
 }
 
+// A pass of one complex128 gate is the same work as the gate alone, whose kernel
+// (mfma.hip) needs no tile: on 4 qubits it is the faster one (20 qubits 8.5 us,
+// 22 qubits 23, 24 qubits 83; the pass 9..12, 27..39, 86..118), on 5 where both
+// lowest bits are targets (24 qubits 109 and 136; others 112 and 110, 20 qubits 14
+// and 10).
+bool pass_pays(int dtype, int n, const ua_gate* gates, int count) {
+  return count > 1 || dtype == UA_COMPLEX64 ||
+         (gates[0].num_targets == 5 && (target_mask(gates[0], n) & 3) != 3);
+}
+
 // One pass of gates[0..count) (4/5-qubit gates) in place.
 int launch_pass(void* state, int dtype, int n, int64_t batch, const ua_gate* gates, int count,
                 bool reverse, hipStream_t s) {
@@ -391,8 +401,13 @@ int launch_pass(void* state, int dtype, int n, int64_t batch, const ua_gate* gat
   // (50 gates, 24 qubits): complex128 4.50 ms staged, 3.77 both ways direct (20
   // qubits 0.92 -> 0.59); complex64 1.97 staged, 1.94 direct in, 2.03 direct
   // out, and in only where the lanes keep runs of 32 bytes.
-  p.direct_in = !c64 || !(target_mask(gates[0], n) & 3);
-  p.direct_out = !c64 && count > 1;
+  // A single complex128 gate only writes directly (5 qubits at 20: 24 us the other
+  // way round, 10 so).  Beyond the Infinity Cache a last gate with both lowest
+  // bits among its targets, which leaves the lanes pieces of lines, goes through
+  // LDS (24 qubits, 2 gates: 1.13 and 0.99 of 123 us).
+  p.direct_in = c64 ? !(target_mask(gates[0], n) & 3) : count > 1;
+  p.direct_out = !c64 && !((target_mask(gates[count - 1], n) & 3) == 3 && count > 1 &&
+                           (batch << n) >= (int64_t(1) << 24));
   for (int gi = 0; gi < count; ++gi) {
     const ua_gate& g = gates[gi];
     BlockGate& b = p.g[gi];
@@ -488,7 +503,8 @@ extern "C" int ua_run_dense_blocks(void* state, int dtype, int num_qubits, int64
     if (events && !(i > 0 && events[2 * i] == events[2 * i - 1])) rc = record_event(events[2 * i], s);
     if (rc) break;
     const Unit& u = units[i];
-    if (u.pass && pass_aligned(state, dtype, gates + u.first, u.count)) {
+    if (u.pass && pass_aligned(state, dtype, gates + u.first, u.count) &&
+        pass_pays(dtype, num_qubits, gates + u.first, u.count)) {
       rc = launch_pass(state, dtype, num_qubits, batch, gates + u.first, u.count, i & 1, s);
     } else {
       for (int j = 0; j < u.count && rc == UA_OK; ++j)

@@ -173,6 +173,36 @@ def test_blocks_misaligned_matrix_runs_gate_by_gate(device):
 
 
 @pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
+@pytest.mark.parametrize("n,batch", [(14, 1), (14, 3), (18, 2)])
+@pytest.mark.parametrize("bits", [(0, 1, 2, 3, 4), (0, 7, 9, 3, 11), (2, 8, 3, 9, 5), (1, 0, 9, 13, 6),
+                                  (0, 1, 2, 3), (4, 9, 2, 11), (13, 12, 11, 10)])
+def test_blocks_of_one_gate(device, dt, n, batch, bits):
+    """A pass of a single gate: its targets on the lowest bits or off them."""
+    rng = np.random.default_rng(n + len(bits))
+    gates = [Gate("dense", tuple(n - 1 - b for b in bits), matrix=haar_unitary(2 ** len(bits), rng))]
+    psi = seeded_state_np(n, (batch,), seed=n)
+    ref = np.stack([oc.run_closed_form(gates, p) for p in psi])
+    got, _ = run_blocks(Circuit(n, gates), psi, dt, device)
+    fe, ma = BAR[dt]
+    assert np.max(U.fidelity_error(ref, got)) < fe and U.max_abs_error(ref, got) < ma
+
+
+def test_blocks_last_gate_on_the_lowest_bits_beyond_the_caches(device):
+    """complex128, 2^24 amplitudes: the last gate of a pass leaves through LDS; the same
+    gates one by one."""
+    n, batch = 16, 256
+    rng = np.random.default_rng(5)
+    gates = [Gate("dense", tuple(n - 1 - b for b in bs), matrix=haar_unitary(2 ** len(bs), rng))
+             for bs in ((5, 9, 3, 12), (1, 7, 0, 11))]
+    g = torch.Generator(device=device).manual_seed(3)
+    x = torch.randn(batch, 2 ** n, generator=g, device=device, dtype=torch.complex128) / 2 ** (n / 2)
+    runners = [CircuitRunner(Circuit(n, gates), dtype=torch.complex128, device=device,
+                             in_place=True, dense_blocks=b) for b in (True, False)]
+    a, b = (r.run(x.clone()) for r in runners)
+    assert float((a - b).abs().max()) < 1e-14
+
+
+@pytest.mark.parametrize("dt", [torch.complex64, torch.complex128])
 @pytest.mark.parametrize("n,batch", [(15, 1), (15, 3), (20, 1), (14, 192)])
 def test_blocks_walk_every_tile_either_way(device, dt, n, batch):
     """Passes that walk the tiles forwards and backwards, 8, 24 and 256 tiles and
