@@ -120,11 +120,14 @@ __device__ __forceinline__ T expmi_phase(float t) {
 }
 #endif
 
-// Loads of phase factors and angles.  Arrays as large as the eight L2s
-// together (32 MB) are read once a pass and never met again in a cache: they
-// are loaded nontemporally, which leaves the state there (24 qubits: a pass
-// with three phases 179 -> 165 us).  Smaller ones stay cached for the other
-// states of a batch.
+// Loads of phase factors.  With complex64 states of 24 qubits and more one array
+// takes half of the Infinity Cache (128 MB), so that what it leaves there is gone
+// before the program's next run and the state is pushed out for it: such arrays
+// are loaded nontemporally (24 qubits, 4 to 20 phases: 0.91..0.96 of the time,
+// with two states 0.85, 25 qubits 0.87).  Smaller ones are met again, by the
+// other states of a batch or by the next run (22 qubits, 4 phases: 1.10 past the
+// caches), complex128 factors gain nothing at any size (1.0..1.17 at 21 to 24
+// qubits), and neither do angles, half as long and waiting for a sincos.
 template <typename V> __device__ __forceinline__ V ldp(const GL V* p) {
 #if UA_STREAM_PHASES
   return __builtin_nontemporal_load(p);
@@ -145,7 +148,7 @@ __device__ __forceinline__ void st2(GL T* p, T a, T b) {
   *reinterpret_cast<GL v2r*>(p) = x; *reinterpret_cast<GL v2r*>(p + 1) = y;
 }
 __device__ __forceinline__ void ld2r(const GL R* p, R& a, R& b) {
-  const v2r x = ldp(reinterpret_cast<const GL v2r*>(p)); a = x.x; b = x.y;
+  const v2r x = *reinterpret_cast<const GL v2r*>(p); a = x.x; b = x.y;
 }
 __device__ __forceinline__ void ld2f(const GL T* p, T& a, T& b) {
   const v2r x = ldp(reinterpret_cast<const GL v2r*>(p));
@@ -164,7 +167,7 @@ __device__ __forceinline__ void st2(GL T* p, T a, T b) {
   *reinterpret_cast<GL v4r*>(p) = x;
 }
 __device__ __forceinline__ void ld2r(const GL R* p, R& a, R& b) {
-  const v2r x = ldp(reinterpret_cast<const GL v2r*>(p)); a = x.x; b = x.y;
+  const v2r x = *reinterpret_cast<const GL v2r*>(p); a = x.x; b = x.y;
 }
 __device__ __forceinline__ void ld2f(const GL T* p, T& a, T& b) {
   const v4r x = ldp(reinterpret_cast<const GL v4r*>(p));
@@ -416,7 +419,7 @@ std::string generate(const PassShape& ps) {
   // of a gradient step, and they round as the interpreted passes do.
   const bool mfma = !dbl && tbits > 12;
   s << "#define UA_DOUBLE " << (dbl ? 1 : 0) << "\n#define UA_MFMA " << (mfma ? 1 : 0)
-    << "\n#define UA_STREAM_PHASES " << (n >= (dbl ? 21 : 22) ? 1 : 0) << "\n" << kPrelude;
+    << "\n#define UA_STREAM_PHASES " << (!dbl && n >= 24 ? 1 : 0) << "\n" << kPrelude;
   // five 12-bit tiles fit a CU's LDS (16 qubits x 1024 states, a gradient step of
   // 30 passes: 21.46 -> 21.27 ms)
   const int waves = dbl ? 2 : g_compiled_waves > 0 ? int(g_compiled_waves) : tbits == 12 ? 5 : 4;

@@ -167,3 +167,25 @@ def test_run_from_a_source_argument_checks():
                    (base, 1), (base + 3 * one - 16, 1), (base - one + 16, 1)):
         assert run(src, m) == _lib.UA_ERR_INVALID_ARGUMENT, (src, m)
     assert run(base + 8 * one, 1, 0) == _lib.UA_OK
+
+
+def _source(code, n, tile_bits):
+    lib = _lib.load()
+    passes, arr = _structs(random_mixed_circuit(n, 20, seed=3), n, tile_bits)
+    buf, length = ctypes.create_string_buffer(1 << 20), ctypes.c_int64()
+    _lib.check(lib.ua_fused_pass_source(code, n, ctypes.byref(passes[0][0]),
+                                        ctypes.c_void_p(passes[0][1]), buf, len(buf),
+                                        ctypes.byref(length)), "source")
+    return buf.value.decode()
+
+
+@pytest.mark.parametrize("code,n,streamed", [(_lib.UA_COMPLEX64, 16, 0), (_lib.UA_COMPLEX64, 22, 0),
+                                             (_lib.UA_COMPLEX64, 23, 0), (_lib.UA_COMPLEX64, 24, 1),
+                                             (_lib.UA_COMPLEX128, 22, 0), (_lib.UA_COMPLEX128, 23, 0)])
+def test_factors_the_caches_can_keep_are_loaded_through_them(code, n, streamed):
+    """Factor arrays that other states or the next run meet again are not loaded
+    past the caches; angles never are."""
+    src = _source(code, n, 13)
+    assert f"#define UA_STREAM_PHASES {streamed}\n" in src
+    angles = src[src.index("void ld2r("):]
+    assert "ldp(" not in angles[:angles.index("}")]
