@@ -24,7 +24,8 @@ them less for each layer of a z-y ansatz).  CZs after the last rotation commute
 with the observable and are left out.  psi and lam are stored as one (2B, 2^n)
 batch, so every inverse step is one fused program over both.  Un-applying gates in complex64 drifts, so psi is
 re-synchronised from checkpoints taken every ceil(sqrt(groups)) groups.
-Memory: two states plus ceil(sqrt(groups)) checkpoints.
+Memory: the final state and up to ceil(sqrt(groups)) - 1 checkpoints between
+forward and backward, and two states more in the backward.
 """
 from __future__ import annotations
 
@@ -371,19 +372,13 @@ class _AdjointExpectation(torch.autograd.Function):
             last_traffic["forward_bytes"] = _bytes(psi)
             ckpt = {}
             # The state before segment c0 stays where it is and the next pass
-            # writes elsewhere, at last into the half of X that the backward
-            # pass works on: no copies (at 16 qubits x 1024 states 0.18 ms
-            # each, three checkpoints, their restores and the copy into X).
-            X = None
-            for i, (c0, prog) in enumerate(progs.fwd):
+            # writes elsewhere: no copies (at 16 qubits x 1024 states 0.18 ms
+            # each, three checkpoints and their restores).
+            for c0, prog in progs.fwd:
                 source = None
                 if c0 > 0:
                     source = ckpt[c0] = psi
-                    if ctx.needs_input_grad[0] and i == len(progs.fwd) - 1:
-                        X = torch.empty(2 * B, 2 ** n, dtype=dtype, device=dev)
-                        psi = X[:B]
-                    else:
-                        psi = torch.empty_like(psi)
+                    psi = torch.empty_like(psi)
                 if prog is not None:
                     _run_counted(prog, psi, "forward_bytes", source)
                 elif source is not None:
@@ -393,13 +388,13 @@ class _AdjointExpectation(torch.autograd.Function):
             loss = _diag_loss(obs, psi)
             last_traffic["forward_bytes"] += _bytes(psi) + _bytes(obs)
         ctx.save_for_backward(params, observable)
-        ctx.state = (spec, dtype, obs, psi, X, ckpt, progs)
+        ctx.state = (spec, dtype, obs, psi, ckpt, progs)
         return loss
 
     @staticmethod
     def backward(ctx, gloss):
         params, observable = ctx.saved_tensors
-        spec, dtype, obs, psi, X, ckpt, progs = ctx.state
+        spec, dtype, obs, psi, ckpt, progs = ctx.state
         ctx.state = None
         n, B, dev = spec.n, params.shape[0], params.device
         lib = _lib.load()
@@ -411,26 +406,24 @@ class _AdjointExpectation(torch.autograd.Function):
                 grad_obs = (w if observable.dim() == 2 else w.sum(0)).to(observable.dtype)
             if not ctx.needs_input_grad[0]:
                 return grad_p, grad_obs, None, None, None
+            # diagonal scaling (read psi and obs, write lambda); the first program
+            # reads psi where the forward left it and writes it beside lambda
+            X = torch.empty(2 * B, 2 ** n, dtype=dtype, device=dev)
             last_traffic["backward_bytes"] = 2 * _bytes(psi) + _bytes(obs)
-            if X is None:                            # one run of segments: no checkpoint
-                X = torch.empty(2 * B, 2 ** n, dtype=dtype, device=dev)
-                X[:B].copy_(psi)
-                last_traffic["backward_bytes"] += 2 * _bytes(psi)
-            # diagonal scaling (read psi and obs, write lambda)
             code = _lib.DTYPE_CODES
             rc = lib.ua_apply_diagonal(_lib.ptr(X[B:]), _lib.ptr(psi), code[dtype],
                                        _lib.ptr(obs), code[obs.dtype],
                                        0 if obs.dim() == 1 else 2 ** n, n, B,
                                        _lib.stream_handle(dev))
             _lib.check(rc, "apply_diagonal")
-            del psi
             ws = torch.empty(lib.ua_pauli_gradients_workspace(n, B), dtype=torch.uint8,
                              device=dev)
             # one (B, n) block of values per (segment, Pauli kind), gathered once at
             # the end: grad[:, idx] += 2 coef vals[block, :, qubit]
             blocks, index = _value_blocks(spec, dev)
             vals = torch.empty(max(1, len(blocks)), B, n, dtype=torch.float64, device=dev)
-            at_psi = X[:B]        # psi at this point: a checkpoint until the next run
+            at_psi = psi          # psi at this point: outside of X until the next run
+            del psi
             for step, what in progs.back:
                 if step == "run":
                     _run_counted(what, X, "backward_bytes",

@@ -223,3 +223,25 @@ def test_pauli_gradients_with_z(device, dtype, tol, n, B):
             # |lambda| and |psi| are about 1: absolute errors
             assert float((z[:, q] - zr.sum((1, 2))).abs().max()) < tol
             assert float((out[:, q] - pr.sum((1, 2))).abs().max()) < tol
+
+
+def test_states_held_for_the_backward(device):
+    """Between forward and backward: the final states and the checkpoints, and no
+    more during a forward that nothing differentiates."""
+    n, B, L = 18, 2, 8                         # 16 segments: checkpoints before 4, 8 and 12
+    gates = adjoint.hardware_efficient_gates(n, L)
+    obs = adjoint.sum_z_observable(n, device)
+    params = torch.rand(B, 2 * n * L, device=device).requires_grad_(True)
+    state = B * 2 ** n * 8
+    adjoint.expectation(params, gates, obs, n).sum().backward()          # tables are made once
+    params.grad = None
+    torch.cuda.synchronize()
+    base = torch.cuda.memory_allocated()
+    loss = adjoint.expectation(params, gates, obs, n)
+    assert torch.cuda.memory_allocated() - base < 4.5 * state
+    del loss
+    base = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    with torch.no_grad():
+        adjoint.expectation(params, gates, obs, n)
+    assert torch.cuda.max_memory_allocated() - base < 4.5 * state
