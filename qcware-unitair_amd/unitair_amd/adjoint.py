@@ -193,8 +193,8 @@ def _value_blocks(spec, dev):
     hit = _GROUP_INDEX.get(key) if spec.key is not None else None
     if hit is None:
         blocks, rows = {}, []
-        for s, (_, rot) in enumerate(spec.segments):
-            for kind, q, idx, coef in rot:
+        for s in reversed(range(len(spec.segments))):       # as the backward meets them
+            for kind, q, idx, coef in spec.segments[s][1]:
                 blk = blocks.setdefault((s, kind), len(blocks))
                 rows.append((blk, q, idx, 2.0 * coef))
         cols = list(zip(*rows)) if rows else [(), (), (), ()]
@@ -419,7 +419,9 @@ class _AdjointExpectation(torch.autograd.Function):
             ws = torch.empty(lib.ua_pauli_gradients_workspace(n, B), dtype=torch.uint8,
                              device=dev)
             # one (B, n) block of values per (segment, Pauli kind), gathered once at
-            # the end: grad[:, idx] += 2 coef vals[block, :, qubit]
+            # the end: grad[idx] += 2 coef vals[block, :, qubit].  index_put_ sorts
+            # the indices and adds what a parameter gets in their order; index_add_
+            # of this many rows adds them atomically, in another order each time
             blocks, index = _value_blocks(spec, dev)
             vals = torch.empty(max(1, len(blocks)), B, n, dtype=torch.float64, device=dev)
             at_psi = psi          # psi at this point: outside of X until the next run
@@ -449,11 +451,11 @@ class _AdjointExpectation(torch.autograd.Function):
                             rc = lib.ua_pauli_gradients(_lib.ptr(vals[blk]), *args)
                         _lib.check(rc, "pauli_gradients")
                         last_traffic["backward_bytes"] += _bytes(X)
-            grad = torch.zeros(B, params.shape[1], dtype=torch.float64, device=dev)
+            grad = torch.zeros(params.shape[1], B, dtype=torch.float64, device=dev)
             if blocks:
                 blk, qs, idx, coef = index
-                grad.index_add_(1, idx, vals[blk, :, qs].transpose(0, 1) * coef)
-            grad_p = (grad * gloss.to(torch.float64).view(B, 1)).to(params.dtype)
+                grad.index_put_((idx,), vals[blk, :, qs] * coef.view(-1, 1), accumulate=True)
+            grad_p = (grad.t().contiguous() * gloss.to(torch.float64).view(B, 1)).to(params.dtype)
         return grad_p, grad_obs, None, None, None
 
 

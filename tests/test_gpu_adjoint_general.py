@@ -245,3 +245,23 @@ def test_states_held_for_the_backward(device):
     with torch.no_grad():
         adjoint.expectation(params, gates, obs, n)
     assert torch.cuda.max_memory_allocated() - base < 4.5 * state
+
+
+@pytest.mark.parametrize("n,layers", [(4, 40), (9, 12)])
+def test_shared_parameters_give_the_same_bits_each_time(device, n, layers):
+    """Parameters used in many groups: their contributions are added in one order."""
+    B, P = 300, 3
+    gates = []
+    for l in range(layers):
+        gates += [("yzx"[l % 3], q, (l + q) % P, 0.3 + 0.01 * (l * n + q)) for q in range(n)]
+        gates += [("cz", q, (q + 1) % n) for q in range(n)]
+    g = torch.Generator(device=device).manual_seed(n)
+    params = torch.rand(B, P, generator=g, device=device, dtype=torch.float64).requires_grad_(True)
+    obs = torch.randn(2 ** n, generator=g, device=device, dtype=torch.float64)
+
+    def grad():
+        loss = adjoint.expectation(params, gates, obs, n, dtype=torch.complex128)
+        return torch.autograd.grad(loss.sum(), params)[0]
+    first = grad()
+    for _ in range(10):
+        assert torch.equal(grad(), first)
