@@ -70,8 +70,7 @@ const char* ua_last_error(void);
  *                       0: vector units for every gate.
  * UA_TUNE_COMPILED_WAVES waves per SIMD that passes compiled afterwards by
  *                       ua_compile_fused_pass ask the register allocator for
- *                       (complex64; 0 = default: 4, for 12-bit tiles 5; else
- *                       1..8); complex128
+ *                       (complex64; 0 = default 4, else 1..8); complex128
  *                       passes always ask for 2. */
 enum { UA_TUNE_UNROLL = 0, UA_TUNE_LANE_EXCHANGE = 1, UA_TUNE_MFMA = 2,
        UA_TUNE_COMPILED_WAVES = 3 };

@@ -40,7 +40,9 @@ constexpr int kMinTileBits = 12;  // tiles below 12 bits stay with the interpret
 int max_tile_bits(int dtype) { return dtype == UA_COMPLEX128 ? 13 : 14; }
 
 // Waves per SIMD the compiled complex64 kernels ask the register allocator
-// for (0: 4, and 5 for 12-bit tiles, whose 32 KiB fit a CU's LDS five times).
+// for (0: 4; a complex64 12-bit tile takes 32 KiB of LDS, so five workgroups of
+// four waves fit a CU, but with 96 registers in place of 128 passes with phases
+// took 1.03 to 1.15 of the time at 14 to 24 qubits and others 0.98 to 1.04).
 // complex128 kernels ask for 2.
 std::atomic<int> g_compiled_waves{0};
 
@@ -420,9 +422,7 @@ std::string generate(const PassShape& ps) {
   const bool mfma = !dbl && tbits > 12;
   s << "#define UA_DOUBLE " << (dbl ? 1 : 0) << "\n#define UA_MFMA " << (mfma ? 1 : 0)
     << "\n#define UA_STREAM_PHASES " << (!dbl && n >= 24 ? 1 : 0) << "\n" << kPrelude;
-  // five 12-bit tiles fit a CU's LDS (16 qubits x 1024 states, a gradient step of
-  // 30 passes: 21.46 -> 21.27 ms)
-  const int waves = dbl ? 2 : g_compiled_waves > 0 ? int(g_compiled_waves) : tbits == 12 ? 5 : 4;
+  const int waves = dbl ? 2 : g_compiled_waves > 0 ? int(g_compiled_waves) : 4;
   s << "extern \"C\" __global__ __launch_bounds__(" << threads
     << ") __attribute__((amdgpu_waves_per_eu("
     << waves << ")))\nvoid ua_compiled_pass(T* __restrict__ state, "

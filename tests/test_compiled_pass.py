@@ -189,3 +189,8 @@ def test_factors_the_caches_can_keep_are_loaded_through_them(code, n, streamed):
     assert f"#define UA_STREAM_PHASES {streamed}\n" in src
     angles = src[src.index("void ld2r("):]
     assert "ldp(" not in angles[:angles.index("}")]
+
+
+def test_default_waves_of_complex64_passes():
+    for tile_bits in (12, 13):
+        assert "amdgpu_waves_per_eu(4)" in _source(_lib.UA_COMPLEX64, 16, tile_bits)
