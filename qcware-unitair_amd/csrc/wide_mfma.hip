@@ -109,7 +109,8 @@ void dense_gemm_kernel(T* out, const T* in, GemmPass p) {
   const T* U = static_cast<const T*>(p.op) + b * p.op_bstride;
 
   // ---- this wavefront's row and group tiles; its first columns of U
-  const int wr = wave % Sh::WR, wc = wave / Sh::WR % Sh::WC, ks = wave / Sh::WR / Sh::WC;
+  const int wr = wave % Sh::WR, wc = KS > 1 ? wave / Sh::WR % Sh::WC : wave / Sh::WR;
+  const int ks = KS > 1 ? wave / Sh::WR / Sh::WC : 0;
   constexpr int KW = KK / KS;            // steps of a wavefront, from kb on
   const int kb = ks * KW;
   const int t0 = (int(blockIdx.y) * Sh::WR + wr) * RTW;
