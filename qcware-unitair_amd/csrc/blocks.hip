@@ -207,8 +207,9 @@ void dense_blocks_kernel(T* state, BlockPass p) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int64_t t = blockIdx.x;
   if (p.group) {  // workgroup t runs on XCD t % 8
-    const int64_t gr = p.group, w = p.reverse ? (p.tiles >> 3) - 1 - (t >> 3) : t >> 3;
-    t = (w / gr) * (8 * gr) + (t & 7) * gr + w % gr;
+    const unsigned gr = p.group, i = blockIdx.x >> 3;
+    const unsigned w = p.reverse ? unsigned(p.tiles >> 3) - 1 - i : i;
+    t = (w / gr) * (8 * gr) + (blockIdx.x & 7) * gr + w % gr;
   } else if (p.reverse) {
     t = p.tiles - 1 - t;
   }
