@@ -184,22 +184,40 @@ def _gates_key(gates, n: int, num_params: int) -> int:
 _GROUP_INDEX = {}
 
 
+# A parameter's contributions are added one after another while it has at most this
+# many (a launch for each round of all parameters); more are sorted by index_put_,
+# which takes about 100 us whatever their number.
+_MAX_ROUNDS = 8
+
+
 def _value_blocks(spec, dev):
-    """{(segment, Pauli kind): block of values} and, for every rotation, device
-    index tensors (block, qubit, parameter index, 2 * coefficient), made once
-    per gate list and device: building them per call would copy from the host,
-    which waits for the stream."""
+    """{(segment, Pauli kind): block of values}, for every rotation, device
+    index tensors (block, qubit, parameter index, 2 * coefficient), and the
+    bounds of runs of rotations that hold each parameter once at most; made
+    once per gate list and device: building them per call would copy from the
+    host, which waits for the stream.  The r-th run holds each parameter's r-th
+    rotation as the backward meets them; one run of all if that takes too many."""
     key = (spec.key, "blocks", str(dev))
     hit = _GROUP_INDEX.get(key) if spec.key is not None else None
     if hit is None:
-        blocks, rows = {}, []
-        for s in reversed(range(len(spec.segments))):       # as the backward meets them
+        blocks, rounds, seen = {}, [], {}
+        for s in reversed(range(len(spec.segments))):
             for kind, q, idx, coef in spec.segments[s][1]:
                 blk = blocks.setdefault((s, kind), len(blocks))
-                rows.append((blk, q, idx, 2.0 * coef))
+                r = min(seen.get(idx, 0), _MAX_ROUNDS)
+                seen[idx] = r + 1
+                if r == len(rounds):
+                    rounds.append([])
+                rounds[r].append((blk, q, idx, 2.0 * coef))
+        rows = [row for part in rounds for row in part]
+        bounds = [0]
+        for part in rounds:
+            bounds.append(bounds[-1] + len(part))
+        if len(rounds) > _MAX_ROUNDS:
+            bounds = None
         cols = list(zip(*rows)) if rows else [(), (), (), ()]
         hit = (blocks, tuple(torch.tensor(c, dtype=torch.int64, device=dev) for c in cols[:3]) +
-               (torch.tensor(cols[3], dtype=torch.float64, device=dev),))
+               (torch.tensor(cols[3], dtype=torch.float64, device=dev).view(-1, 1),), bounds)
         if spec.key is not None:
             if len(_GROUP_INDEX) >= 4 * _TEMPLATE_LIMIT:
                 _GROUP_INDEX.pop(next(iter(_GROUP_INDEX)))
@@ -419,10 +437,8 @@ class _AdjointExpectation(torch.autograd.Function):
             ws = torch.empty(lib.ua_pauli_gradients_workspace(n, B), dtype=torch.uint8,
                              device=dev)
             # one (B, n) block of values per (segment, Pauli kind), gathered once at
-            # the end: grad[idx] += 2 coef vals[block, :, qubit].  index_put_ sorts
-            # the indices and adds what a parameter gets in their order; index_add_
-            # of this many rows adds them atomically, in another order each time
-            blocks, index = _value_blocks(spec, dev)
+            # the end: grad[idx] += 2 coef vals[block, :, qubit]
+            blocks, index, bounds = _value_blocks(spec, dev)
             vals = torch.empty(max(1, len(blocks)), B, n, dtype=torch.float64, device=dev)
             at_psi = psi          # psi at this point: outside of X until the next run
             del psi
@@ -451,10 +467,17 @@ class _AdjointExpectation(torch.autograd.Function):
                             rc = lib.ua_pauli_gradients(_lib.ptr(vals[blk]), *args)
                         _lib.check(rc, "pauli_gradients")
                         last_traffic["backward_bytes"] += _bytes(X)
+            # (index_add_ of rows that share a parameter adds them atomically, in
+            # another order each time)
             grad = torch.zeros(params.shape[1], B, dtype=torch.float64, device=dev)
             if blocks:
                 blk, qs, idx, coef = index
-                grad.index_put_((idx,), vals[blk, :, qs] * coef.view(-1, 1), accumulate=True)
+                rows = vals[blk, :, qs] * coef
+                if bounds is None:
+                    grad.index_put_((idx,), rows, accumulate=True)
+                else:
+                    for r0, r1 in zip(bounds, bounds[1:]):
+                        grad.index_add_(0, idx[r0:r1], rows[r0:r1])
             grad_p = (grad.t().contiguous() * gloss.to(torch.float64).view(B, 1)).to(params.dtype)
         return grad_p, grad_obs, None, None, None
 

@@ -265,3 +265,25 @@ def test_shared_parameters_give_the_same_bits_each_time(device, n, layers):
     first = grad()
     for _ in range(10):
         assert torch.equal(grad(), first)
+
+
+@pytest.mark.parametrize("P,layers", [(36, 2), (24, 2), (7, 2), (6, 8), (1, 3)])
+def test_parameters_used_once_a_few_times_and_often(device, P, layers):
+    """One run of additions, several, and more than are made one after another."""
+    n, B = 6, 2
+    gates = [(("y", "z", "x")[k], q, (l * 3 * n + k * n + q) % P, 0.4 + 0.02 * q)
+             for l in range(layers) for k in range(3) for q in range(n)]
+    rng = np.random.default_rng(P)
+    params = rng.uniform(-np.pi, np.pi, (B, P))
+    obs = rng.standard_normal(2 ** n)
+    _, g, _ = _run(device, params, gates, obs, n, torch.complex128)
+    h = 1e-5
+    for i in range(P):
+        up, down = params.copy(), params.copy()
+        up[:, i] += h
+        down[:, i] -= h
+        for b in range(B):
+            cd = (AO.general_loss(up[b], gates, obs, n) -
+                  AO.general_loss(down[b], gates, obs, n)) / (2 * h)
+            # O(h^2) of the third derivative (up to uses * 0.52 to the third), 1e-16 / h
+            assert abs(g[b, i] - cd) < 1e-6, (b, i)
