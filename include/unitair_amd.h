@@ -62,12 +62,20 @@ const char* ua_last_error(void);
  * UA_TUNE_LANE_EXCHANGE 1 (default): 1-qubit gates on index bits 1..6 move
  *                       contiguous amplitude pairs and exchange partners
  *                       across lanes; 0: strided pair access.
- * UA_TUNE_MFMA          1 (default): complex gates with one operator for the
- *                       batch run on the matrix cores (v_mfma_f32/f64_16x16x4)
- *                       when k = 5, when k = 4 in complex128, and when k = 4
- *                       in complex64 with every target on index bits 0..5 or
- *                       at most 2^22 amplitudes in the batch;
- *                       0: vector units for every gate.
+ * UA_TUNE_MFMA          1 (default): single complex gates (ua_apply_operator,
+ *                       the gates of ua_run_circuit, gates that
+ *                       ua_run_dense_blocks runs by themselves) use the matrix
+ *                       cores (v_mfma_f32/f64_16x16x4) where they are faster.
+ *                       With one operator for the batch: k = 5; k = 4 in
+ *                       complex128; k = 4 in complex64 with every target on
+ *                       index bits 0..5 or at most 2^22 amplitudes in the batch
+ *                       (2^21 with a target on bit 0).  With one operator or one
+ *                       per state, states of at least 12 qubits and memory
+ *                       aligned to two elements: k = 6..10 (complex128 6..9),
+ *                       but for complex64 k = 7 and 8 in place with one operator.
+ *                       0: vector units for these gates.  1-qubit layers, passes
+ *                       of compiled programs and of dense blocks, and operator
+ *                       gradients use the matrix cores whatever the value.
  * UA_TUNE_COMPILED_WAVES waves per SIMD that passes compiled afterwards by
  *                       ua_compile_fused_pass ask the register allocator for
  *                       (complex64; 0 = default 4, else 1..8); complex128

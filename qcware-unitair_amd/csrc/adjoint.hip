@@ -586,17 +586,17 @@ int pauli_gradients(double* out, double* z_out, const void* lambda, const void* 
     if (pauli == UA_PAULI_X) {                                                                 \
       if (c64)                                                                                 \
         grad_high_kernel<float2, UA_PAULI_X, HH><<<grid, kBlock, 0, s>>>(                      \
-            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);                \
+            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);        \
       else                                                                                     \
         grad_high_kernel<double2, UA_PAULI_X, HH><<<grid, kBlock, 0, s>>>(                     \
-            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);              \
+            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);      \
     } else {                                                                                   \
       if (c64)                                                                                 \
         grad_high_kernel<float2, UA_PAULI_Y, HH><<<grid, kBlock, 0, s>>>(                      \
-            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);                \
+            part, (const float2*)lambda, (const float2*)psi, n, w0, per_block, chunks);        \
       else                                                                                     \
         grad_high_kernel<double2, UA_PAULI_Y, HH><<<grid, kBlock, 0, s>>>(                     \
-            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);              \
+            part, (const double2*)lambda, (const double2*)psi, n, w0, per_block, chunks);      \
     }                                                                                          \
   }
     UA_HIGH(1) UA_HIGH(2) UA_HIGH(3) UA_HIGH(4)
@@ -744,14 +744,18 @@ extern "C" int ua_expect_sum_z(double* out, const void* psi, int dtype, int num_
 // products in float64 registers, and the workgroup reduces them with
 // wavefront shuffles and LDS.  With one part the sums go straight to grad_op;
 // otherwise to the float64 workspace, and op_grad_finish_kernel adds the
-// parts (one workgroup per result entry).  k = 1, 2 take the whole result in one block (each amplitude read
-// once); larger k tile it 4 x 4 (most operators on 4 and 5 qubits:
-// op_grad_mfma_kernel).
+// parts (one workgroup per result entry).  k = 1, 2 take the whole result in
+// one block (each amplitude read once); larger k tile it 4 x 4, unless
+// op_grad_on_mfma prefers op_grad_mfma_kernel.
 //
 // GS (k = 1, 2): the thread holds whole groups of grad_out, so it also forms the
 // state's gradient U^H grad_out of them: one read of grad_out less, and no
 // adjoint operator to make first (22 qubits x 3 states, k = 2, forward and
-// backward: 195 -> 153 us, of which the kernels are about 100).
+// backward: 195 -> 153 us, of which the kernels are about 100).  In complex128 with
+// a target on bit 0 and 2^15 to 2^18 amplitudes the one kernel takes longer than the
+// two it replaces (16 qubits, bits 0 and 1: 25.4 and 21.9 us with what makes the
+// adjoint operator), but its call less on the host (89 and 111 us for the whole
+// backward there).
 namespace ua {
 namespace {
 

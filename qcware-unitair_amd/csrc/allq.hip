@@ -151,7 +151,8 @@ struct AllqPass {
 // STAGED: the one stage's cubes would split the lines of memory (plan_layer), so
 // the tile moves in whole lines and LDS lies on both sides of the stage.
 template <typename T, int TB, bool STAGED>
-__global__ __launch_bounds__((1 << TB) / kCube) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 2)))
+__global__ __launch_bounds__((1 << TB) / kCube)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 4 : 2)))
 void allq_pass_kernel(T* out, const T* in, const T* __restrict__ op, AllqPass a) {
   constexpr int kTile = 1 << TB;
   __shared__ T tile[kTile];

@@ -201,7 +201,8 @@ template <typename T, int THREADS>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 8 ? 5 : 2)))
 void dense_blocks_kernel(T* state, BlockPass p) {
   constexpr int UPT = kTile / 2 / THREADS;  // element pairs per thread
-  constexpr int EB = THREADS == 128 ? 8 : 9;  // tile bits of 2 * thread
+  constexpr int EB = 9;                     // tile bits of 2 * thread
+  static_assert(2 * THREADS == 1 << EB, "element pairs");
   constexpr bool kOut = sizeof(T) == 16;
   __shared__ T tile[kTile];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;

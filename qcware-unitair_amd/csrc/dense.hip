@@ -515,8 +515,10 @@ int apply_operator_impl(void* out, const void* state, const void* op, int dtype,
     return check_launch("dense_fast_kernel");
   }
 
-  // (7- and 8-qubit complex64 gates with one operator keep the vector kernel
-  // when they run in place: its rounding there is relied on)
+  // 7- and 8-qubit complex64 gates with one operator keep the vector kernel when
+  // they run in place.  Not for speed (22 qubits 86 and 294 us; out of place on the
+  // matrix cores 43 and 80): their in-place results have always been the vector
+  // kernel's to the bit, and tests/test_gpu_parity.py holds them to that.
   const bool vector_in_place =
       in_place && op_bstride == 0 && dtype == UA_COMPLEX64 && (k == 7 || k == 8);
   if (g_use_mfma && !vector_in_place &&

@@ -77,7 +77,8 @@ template <typename T, int K, int LG, int RTW, int WR_ = 0, int KS = 1> struct Ge
   static constexpr int CTW = CT / WC;
   static constexpr int S = RT / (WR * RTW);   // row slices (blockIdx.y)
   static constexpr int AC = 32 / sizeof(T);   // columns of U a lane reads a step: 32 bytes
-  // workgroups per CU that the registers must leave room for (LDS: 160 KB)
+  // workgroups per CU that the registers must leave room for (LDS: 160 KB; three or
+  // four of 32 KB are within 1 % of each other, 6 and 7 targets, 18 to 24 qubits)
   static constexpr int kLds = sizeof(T) << TB;
   static constexpr int kPerCu = kLds <= 32768 ? (K == 7 ? 4 : 3) : kLds <= 65536 ? 2 : 1;
   // 8-qubit complex64 gates sum 512 real terms as four partial sums of 128 (error
@@ -420,7 +421,7 @@ int apply_dense_gemm(void* out, const void* in, const void* op, int dtype, int n
     default: return split ? launch_gemm<float2, 10, 4, 1>(a) : launch_gemm<float2, 10, 4, 8>(a);
   }
   switch (k) {
-    case 6: return launch_gemm<double2, 6, 5, 1>(a);
+    case 6: return launch_gemm<double2, 6, 5, 1>(a);  // 4 x 2 tiles: one for each wavefront
     case 7: return split ? launch_gemm<double2, 7, 5, 1, 4>(a) : launch_gemm<double2, 7, 5, 1>(a);
     case 8: return split ? launch_gemm<double2, 8, 4, 1>(a) : launch_gemm<double2, 8, 4, 2>(a);
     default: return split ? launch_gemm<double2, 9, 4, 1>(a) : launch_gemm<double2, 9, 4, 4>(a);

@@ -22,8 +22,9 @@ it, because Z commutes with them: it then shares the point of the group before,
 and its inverse is part of that step (one pass over the states and one read of
 them less for each layer of a z-y ansatz).  CZs after the last rotation commute
 with the observable and are left out.  psi and lam are stored as one (2B, 2^n)
-batch, so every inverse step is one fused program over both.  Un-applying gates in complex64 drifts, so psi is
-re-synchronised from checkpoints taken every ceil(sqrt(groups)) groups.
+batch, so every inverse step is one fused program over both.  Un-applying
+gates in complex64 drifts, so psi is re-synchronised from checkpoints taken
+every ceil(sqrt(groups)) groups.
 Memory: the final state and up to ceil(sqrt(groups)) - 1 checkpoints between
 forward and backward, and two states more in the backward.
 """
